@@ -46,6 +46,9 @@ UNITS = [
     ("march3d.hip", "march3d_fast.o", ["-DPPK_NS=fast", "-ffp-contract=fast"]),
     ("march3d.hip", "march3d_strict.o",
      ["-DPPK_NS=strict", "-DPPK_EXACT_DIV", "-ffp-contract=off"]),
+    ("march2d.hip", "march2d_fast.o", ["-DPPK_NS=fast", "-ffp-contract=fast"]),
+    ("march2d.hip", "march2d_strict.o",
+     ["-DPPK_NS=strict", "-DPPK_EXACT_DIV", "-ffp-contract=off"]),
     ("batch.hip", "batch_fast.o", ["-DPPK_NS=fast", "-ffp-contract=fast"]),
     ("batch.hip", "batch_strict.o", ["-DPPK_NS=strict", "-DPPK_EXACT_DIV", "-ffp-contract=off"]),
     # the network's accumulators in VGPRs (no copies out of AGPRs before each ReLU)

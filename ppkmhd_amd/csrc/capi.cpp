@@ -31,7 +31,7 @@ const KernelTable kFast = {fast::staged_boundaries, fast::staged_prim_dt,
                            fast::staged_end,        fast::staged_godunov,
                            fast::fused_godunov,     fast::fused_cfl,
                            fast::fused_half,        fast::surrogate_dump,
-                           fast::surrogate_dump_slots, fast::march_godunov,
+                           fast::surrogate_dump_slots, fast::march_godunov, fast::march2d_godunov,
                            fast::batch_block_counts,
                            fast::batch_step};
 const KernelTable kStrict = {strict::staged_boundaries, strict::staged_prim_dt,
@@ -39,7 +39,7 @@ const KernelTable kStrict = {strict::staged_boundaries, strict::staged_prim_dt,
                              strict::staged_end,        strict::staged_godunov,
                              strict::fused_godunov,     strict::fused_cfl,
                              strict::fused_half,        strict::surrogate_dump,
-                             strict::surrogate_dump_slots, strict::march_godunov,
+                             strict::surrogate_dump_slots, strict::march_godunov, strict::march2d_godunov,
                              strict::batch_block_counts,
                              strict::batch_step};
 
@@ -64,6 +64,20 @@ bool fused_supported(const DevParams &p, int precision, int kernel_path) {
   (void)p;
   if (kernel_path == PPK_PATH_STAGED) return false;
   return precision == PPK_FP64 || precision == PPK_FP64_STRICT || precision == PPK_FP32_BULK;
+}
+
+void march2d_shape(DevParams &p, int cus) {
+  double best = 0.0;
+  for (int lw = 64; lw >= 32; lw /= 2)
+    for (int rows = 1; rows <= p.ny; ++rows) {
+      const double t = march2d_time((double)march2d_waves(p, lw, rows), rows, cus);
+      if (best == 0.0 || t < best * 0.999) {
+        best = t;
+        p.march_lw = lw;
+        p.march_rows = rows;
+      }
+    }
+  p.march = (int)march2d_waves(p, p.march_lw, p.march_rows);
 }
 
 }  // namespace ppk
@@ -251,8 +265,9 @@ int launch_step(ppk_mhd_t *h, double dt, int dt_mode, int check_finished) {
       h->nparts = ppk::fused_cfl_parts(p);
     }
     HIP_CHECK(h, K.set_dt(h->ctrl, h->parts, h->nparts, dt, mode, h->p.cfl, s));
-    if (march) {  // the single-pass 3D step
-      HIP_CHECK(h, K.march_godunov(p, in, out, h->parts, h->ctrl, cfl ? 1 : 0, s, tm));
+    if (march) {  // the single-pass step
+      HIP_CHECK(h, (p.dim == 3 ? K.march_godunov : K.march2d_godunov)(p, in, out, h->parts, h->ctrl,
+                                                                      cfl ? 1 : 0, s, tm));
       if (cfl) h->nparts = (int)ppk::march_blocks(p);
     } else {
       HIP_CHECK(h, K.fused_godunov(p, in, out, h->fw, h->parts, h->ctrl, cfl ? 1 : 0, s, tm));
@@ -343,16 +358,19 @@ int ppk_mhd_create(const ppk_mhd_params *params, ppk_mhd_t **handle) {
   h->K = params->precision == PPK_FP64_STRICT ? &ppk::kStrict : &ppk::kFast;
   h->dp.bulk32 = params->precision == PPK_FP32_BULK ? 1 : 0;
   h->fused = ppk::fused_supported(h->dp, params->precision, params->kernel_path);
-  // FP64 3D: the single-pass kernel, unless the three-kernel form is asked for (the FP32-bulk
+  // FP64: the single-pass kernels, unless the three-kernel form is asked for (the FP32-bulk
   // form and the surrogate run the three-kernel form)
   int dev = 0, cus = 0;
   if (hipGetDevice(&dev) != hipSuccess ||
       hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
     cus = 0;
-  h->dp.march = (params->dim == 3 && h->fused && params->precision != PPK_FP32_BULK &&
-                 params->kernel_path != PPK_PATH_FUSED_RECORDS)
-                    ? ppk::march_nblk(h->dp, cus)
-                    : 0;
+  if (h->fused && params->precision != PPK_FP32_BULK &&
+      params->kernel_path != PPK_PATH_FUSED_RECORDS) {
+    if (params->dim == 3)
+      h->dp.march = ppk::march_nblk(h->dp, cus);
+    else
+      ppk::march2d_shape(h->dp, cus);
+  }
   if (params->kernel_path == PPK_PATH_FUSED && !h->fused) {
     delete h;
     return fail(nullptr, PPK_ERR_UNSUPPORTED, "fused kernels do not support these parameters");

@@ -168,6 +168,29 @@ inline int march_nblk(const DevParams &p, int cus) {
   if (b > total / 16) b = total / 16;
   return (int)(b < 1 ? 1 : b);
 }
+// The single-pass 2D step (march2d.hip): strips of lw - 4 output columns (lw = 64 or 32 lanes)
+// by `rows` output rows, 64 / lw strips per wave; one CFL partial per wave
+inline long long march2d_waves(const DevParams &p, int lw, int rows) {
+  const long long strips = (long long)((p.nx + lw - 5) / (lw - 4)) * ((p.ny + rows - 1) / rows);
+  return (strips + 64 / lw - 1) / (64 / lw);
+}
+// Relative time of a launch of `waves` strips of `rows` output rows.  A strip takes rows + 2
+// passes and a start of about one more.  One wave per SIMD issues instructions in 9 of 10
+// cycles, so a second wave on the same SIMD hides the start but little else: two take 1.9 times
+// as long as one, and so on per further wave.  Few rows give many waves but more passes per
+// row.  Measured (us per launch, MI355X, Orszag-Tang; strips of 64 columns):
+//   64^2    1 row 17.7, 2 rows 22.8, 3 rows 27.8        (128, 64, 44 waves)
+//   256^2   1 row 27.4, 2 rows 24.3, 4 rows 34.1        (1280, 640, 320)
+//   1024^2  8 rows 130, 10 rows 108, 20 rows 121, 32 rows 179  (2304, 1854, 936, 576)
+//   2048^2  24 rows 362, 32 rows 448, 36 rows 361, 64 rows 563 (3010, 2240, 1995, 1120)
+// 32-column strips (two per wave) were within 3 % of these; they pay where 64 columns leave
+// lanes idle, which the wave count shows.
+inline double march2d_time(double waves, int rows, int cus) {
+  const double simds = 4.0 * (cus > 0 ? cus : 256);
+  const double per = waves <= simds ? 1.0 : (double)(long long)((waves + simds - 1.0) / simds);
+  return per <= 1.0 ? rows + 3.1 : 0.93 * per * (rows + 1.6);
+}
+void march2d_shape(DevParams &p, int cus);  // sets march_lw, march_rows and march
 inline long long march_blocks(const DevParams &p) { return p.march > 0 ? p.march : 0; }
 
 // half-step tile shapes of a batch (batch_block_counts / batch_step `tile`): 2D 32x8, 64x4,
@@ -227,6 +250,9 @@ struct BatchMember {
      fill's copy target); CFL partials, one per block, when fold_cfl */                         \
   hipError_t march_godunov(const DevParams &p, const double *Uin, double *Uout, double *parts,   \
                            const double *ctrl, int fold_cfl, hipStream_t s, StageTimer *tm);    \
+  /* the same in 2D: CFL partials, one per wave */                                             \
+  hipError_t march2d_godunov(const DevParams &p, const double *Uin, double *Uout, double *parts, \
+                             const double *ctrl, int fold_cfl, hipStream_t s, StageTimer *tm);  \
   /* batched ensemble: counts of blocks per stage for one member, then the batched step */      \
   void batch_block_counts(const DevParams &p, int tile, long long counts[BS_COUNT]);            \
   hipError_t batch_step(const BatchMember *members, int nmembers, int dim, int bulk32, int tile, \
@@ -250,6 +276,7 @@ struct KernelTable {
   decltype(&fast::surrogate_dump) surrogate_dump;
   decltype(&fast::surrogate_dump_slots) surrogate_dump_slots;
   decltype(&fast::march_godunov) march_godunov;
+  decltype(&fast::march2d_godunov) march2d_godunov;
   decltype(&fast::batch_block_counts) batch_block_counts;
   decltype(&fast::batch_step) batch_step;
 };

@@ -40,7 +40,8 @@ struct DevParams {
   int tile3;            // 3D half-step tile shape (batch tables; 0 for single grids)
   int brick;            // block-to-cells shape of the fused per-cell kernels (batch tables)
   int bulk32;           // FP32-bulk form: half step, records, face/edge solves in float
-  int march;            // 3D single-pass step: blocks of its launch (0: not used)
+  int march;            // single-pass step: blocks (3D) or waves (2D) of its launch (0: not used)
+  int march_lw, march_rows;  // 2D single-pass step: columns (lanes) and output rows of a strip
 };
 
 template <class R>
