@@ -35,51 +35,44 @@ PPK_HD int find_member(const BatchMember *__restrict__ m, int nm, int st, long l
 __device__ __forceinline__ bool member_active(const BatchMember &m) {
   return m.ctrl[CTRL_ACTIVE] != 0.0;
 }
+// parity of the member's current state: the prologue notes it in the control block's spare
+// slot, so that the step's last kernel may count the iteration up
 __device__ __forceinline__ int parity(const BatchMember &m) {
-  return ((long long)m.ctrl[CTRL_ITER]) & 1;
+  return m.ctrl[CTRL_SPARE] != 0.0 ? 1 : 0;
 }
 
-// ---- per-member control: finished() test (SolverBase.cpp:195-201), dt, end of step ---------
-__global__ void k_bbegin(const BatchMember *__restrict__ mem, int nm) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= nm) return;
-  double *ctrl = mem[i].ctrl;
-  const bool done = ctrl[CTRL_T] >= (ctrl[CTRL_TEND] - 1e-14) || ctrl[CTRL_ITER] >= ctrl[CTRL_NSTEPMAX];
-  ctrl[CTRL_ACTIVE] = done ? 0.0 : 1.0;
+// ---- prologue: blocks [0, nm) decide whether their member's step runs (SolverBase.cpp:195-201)
+// and set its dt (unless a standalone CFL pass follows), the others fill the ghosts of the
+// current states, every face, edge and corner in one pass.  They decide for themselves from t
+// and the iteration, which no block of this launch writes.
+__global__ void __launch_bounds__(kBlock) k_bprologue(const BatchMember *__restrict__ mem, int nm,
+                                                      int set_dt) {
+  __shared__ double red[kBlock / 64];
+  if ((int)blockIdx.x < nm) {
+    const BatchMember &m = mem[blockIdx.x];
+    const bool on = step_wanted(m.ctrl, 1);
+    if (threadIdx.x == 0) {
+      m.ctrl[CTRL_ACTIVE] = on ? 1.0 : 0.0;
+      m.ctrl[CTRL_SPARE] = (double)(((long long)m.ctrl[CTRL_ITER]) & 1);
+    }
+    if (on && set_dt)
+      step_dt<kBlock>(m.ctrl, m.parts, m.nparts, 0.0, SETDT_CFL, m.p.cfl, red);
+    return;
+  }
+  const long long gb = (long long)blockIdx.x - nm;
+  const BatchMember &m = mem[find_member(mem, nm, BS_BND, gb)];
+  if (!step_wanted(m.ctrl, 1)) return;
+  const long long t = (gb - m.begin[BS_BND]) * kBlock + threadIdx.x;
+  const int par = ((long long)m.ctrl[CTRL_ITER]) & 1;
+  if (t < ghost_shell_cells(m.p)) ghost_shell_element(m.U[par], m.p, t, nullptr);
 }
 
-// one block per member: reduce its CFL partials, dt = cfl / max, clamped to tEnd - t
+// one block per member: dt = cfl / max of its CFL partials, clamped to tEnd - t
 __global__ void __launch_bounds__(kBlock) k_bset_dt(const BatchMember *__restrict__ mem) {
   __shared__ double red[kBlock / 64];
   const BatchMember &m = mem[blockIdx.x];
-  double *ctrl = m.ctrl;
-  if (ctrl[CTRL_ACTIVE] == 0.0) return;
-  double mx = 0.0;
-  for (int b = threadIdx.x; b < m.nparts; b += kBlock) mx = fmax(mx, m.parts[b]);
-  mx = block_max(mx, red);
-  if (threadIdx.x != 0) return;
-  ctrl[CTRL_INVDT] = mx;
-  double dt = m.p.cfl / mx;
-  if (ctrl[CTRL_T] + dt > ctrl[CTRL_TEND]) dt = ctrl[CTRL_TEND] - ctrl[CTRL_T];
-  ctrl[CTRL_DT] = dt;
-}
-
-__global__ void k_bend(const BatchMember *__restrict__ mem, int nm) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= nm) return;
-  double *ctrl = mem[i].ctrl;
-  if (ctrl[CTRL_ACTIVE] == 0.0) return;
-  ctrl[CTRL_ITER] += 1.0;
-  ctrl[CTRL_T] += ctrl[CTRL_DT];
-}
-
-// ---- ghost fill of the current state, every face, edge and corner in one pass -------------
-__global__ void __launch_bounds__(kBlock) k_bbnd(const BatchMember *__restrict__ mem, int nm) {
-  const long long gb = blockIdx.x;
-  const BatchMember &m = mem[find_member(mem, nm, BS_BND, gb)];
   if (!member_active(m)) return;
-  const long long t = (gb - m.begin[BS_BND]) * kBlock + threadIdx.x;
-  if (t < ghost_shell_cells(m.p)) ghost_shell_element(m.U[parity(m)], m.p, t, nullptr);
+  step_dt<kBlock>(m.ctrl, m.parts, m.nparts, 0.0, SETDT_CFL, m.p.cfl, red);
 }
 
 // ---- standalone CFL partials of the current state ------------------------------------------
@@ -196,6 +189,7 @@ __global__ void __launch_bounds__(kCflBlock) k_bupdate(const BatchMember *__rest
   const double dt = m.ctrl[CTRL_DT];
   const double dtdx = dt / p.dx, dtdy = dt / p.dy, dtdz = DIM == 3 ? dt / p.dz : 0.0;
   const int par = parity(m);
+  if (L == 0 && threadIdx.x == 0) step_end(m.ctrl, nullptr);
   int i, j, k;
   double best = 0.0;
   if (brick_cell(m.pad, L, threadIdx.x, i, j, k))
@@ -234,8 +228,8 @@ void batch_block_counts(const DevParams &p, int tile, long long counts[BS_COUNT]
   counts[BS_UPDATE] = fused_cfl_parts(p);
 }
 
-// one step of every member: finished test, ghost fill, (standalone CFL on request), dt, the
-// three fused stages, end of step.  Stream-ordered, no host synchronization, no memset: safe
+// one step of every member: prologue (finished test, ghost fill, dt), on request a standalone
+// CFL pass and dt from it, the three fused stages (the last one ends the step).  Stream-ordered, no host synchronization, no memset: safe
 // to capture in a graph and replay.
 template <class R>
 void launch_bhalf(const BatchMember *members, int nm, int dim, int tile, long long blocks,
@@ -282,20 +276,18 @@ void launch_rest(const BatchMember *members, int nm, int dim, int tile,
 hipError_t batch_step(const BatchMember *members, int nm, int dim, int bulk32, int tile,
                       const long long totals[BS_COUNT], int with_cfl, hipStream_t s) {
   using namespace batchk;
-  const dim3 b(kBlock), bm((nm + 63) / 64 * 64 > 1024 ? 1024 : (nm + 63) / 64 * 64);
-  const dim3 gm((nm + (int)bm.x - 1) / (int)bm.x);
-  hipLaunchKernelGGL(k_bbegin, gm, bm, 0, s, members, nm);
-  if (totals[BS_BND] > 0)
-    hipLaunchKernelGGL(k_bbnd, dim3((unsigned)totals[BS_BND]), b, 0, s, members, nm);
-  if (with_cfl)
+  const dim3 b(kBlock);
+  hipLaunchKernelGGL(k_bprologue, dim3((unsigned)(nm + totals[BS_BND])), b, 0, s, members, nm,
+                     with_cfl ? 0 : 1);
+  if (with_cfl) {
     hipLaunchKernelGGL(k_bcfl, dim3((unsigned)totals[BS_CFL]), dim3(kCflBlock), 0, s, members,
                        nm);
-  hipLaunchKernelGGL(k_bset_dt, dim3(nm), b, 0, s, members);
+    hipLaunchKernelGGL(k_bset_dt, dim3(nm), b, 0, s, members);
+  }
   if (bulk32)
     launch_rest<float>(members, nm, dim, tile, totals, s);
   else
     launch_rest<double>(members, nm, dim, tile, totals, s);
-  hipLaunchKernelGGL(k_bend, gm, bm, 0, s, members, nm);
   return hipGetLastError();
 }
 

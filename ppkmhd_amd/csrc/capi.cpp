@@ -26,7 +26,7 @@ namespace {
 thread_local std::string g_thread_error;
 
 }  // namespace
-const KernelTable kFast = {fast::staged_boundaries, fast::staged_prim_dt,
+const KernelTable kFast = {fast::staged_boundaries, fast::staged_prologue, fast::staged_prim_dt,
                            fast::staged_begin,      fast::staged_set_dt,
                            fast::staged_end,        fast::staged_godunov,
                            fast::fused_godunov,     fast::fused_cfl,
@@ -34,7 +34,8 @@ const KernelTable kFast = {fast::staged_boundaries, fast::staged_prim_dt,
                            fast::surrogate_dump_slots, fast::march_godunov, fast::march2d_godunov,
                            fast::batch_block_counts,
                            fast::batch_step};
-const KernelTable kStrict = {strict::staged_boundaries, strict::staged_prim_dt,
+const KernelTable kStrict = {strict::staged_boundaries, strict::staged_prologue,
+                             strict::staged_prim_dt,
                              strict::staged_begin,      strict::staged_set_dt,
                              strict::staged_end,        strict::staged_godunov,
                              strict::fused_godunov,     strict::fused_cfl,
@@ -90,7 +91,14 @@ struct ppk_mhd_solver {
   double *U[2] = {nullptr, nullptr};
   double *Q = nullptr;
   double *ctrl = nullptr;       // device control block
-  double *ctrl_host = nullptr;  // pinned mirror (CTRL_SLOTS) + one diagnostics slot
+  double *ctrl_host = nullptr;  // pinned: the control block as the host last read or wrote it
+                                // (CTRL_SLOTS), one diagnostics slot, then the mirror
+  // The fused steps' last kernel writes t, dt, CFL maximum and iteration to this pinned block
+  // too, so that reading them after a step takes a synchronization and no copy.  `mirrored`:
+  // the mirror equals the device block once the stream has drained (false after work that
+  // changes the device block alone).
+  double *mirror = nullptr;
+  bool mirrored = false;
   double *diag = nullptr;       // diagnostics scratch (device)
   double *parts = nullptr;      // per-block CFL partial maxima (device)
   ppk::StagedScratch w;
@@ -218,17 +226,30 @@ ppk::DevParams make_dev(const ppk_mhd_params &p) {
   return d;
 }
 
+constexpr int kMirrored[4] = {ppk::CTRL_T, ppk::CTRL_DT, ppk::CTRL_INVDT, ppk::CTRL_ITER};
+
+// the host's block to the device (synchronizes)
 int write_ctrl(ppk_mhd_t *h) {
   HIP_CHECK(h, hipMemcpyAsync(h->ctrl, h->ctrl_host, sizeof(double) * ppk::CTRL_SLOTS,
                               hipMemcpyHostToDevice, h->stream));
   HIP_CHECK(h, hipStreamSynchronize(h->stream));
+  for (int i : kMirrored) h->mirror[i] = h->ctrl_host[i];
+  h->mirrored = true;
   return PPK_OK;
 }
 
+// the device's block to the host (synchronizes)
 int read_ctrl(ppk_mhd_t *h) {
+  if (h->mirrored) {
+    HIP_CHECK(h, hipStreamSynchronize(h->stream));
+    for (int i : kMirrored) h->ctrl_host[i] = h->mirror[i];
+    return PPK_OK;
+  }
   HIP_CHECK(h, hipMemcpyAsync(h->ctrl_host, h->ctrl, sizeof(double) * ppk::CTRL_SLOTS,
                               hipMemcpyDeviceToHost, h->stream));
   HIP_CHECK(h, hipStreamSynchronize(h->stream));
+  for (int i : kMirrored) h->mirror[i] = h->ctrl_host[i];
+  h->mirrored = true;
   return PPK_OK;
 }
 
@@ -253,34 +274,41 @@ int launch_step(ppk_mhd_t *h, double dt, int dt_mode, int check_finished) {
   ppk::StageTimer *tm = h->tm();
   const bool cfl = dt_mode == PPK_DT_CFL;
   const int mode = cfl ? ppk::SETDT_CFL : ppk::SETDT_FIXED;
-  HIP_CHECK(h, K.begin(h->ctrl, check_finished, s));
-  // the single-pass step writes only the interior of its output: the ghost fill gives the
-  // output the filled input's ghosts (the reference's U2 = U copy) in the same pass
-  const bool march = h->fused && p.march > 0 && !h->fw.sur;
-  HIP_CHECK(h, K.boundaries(p, in, march ? out : nullptr, h->ctrl, s, tm));
-  if (h->fused) {
-    // the previous fused step left the CFL maxima of its output (= in) in parts
-    if (cfl && !h->cfl_valid) {
-      HIP_CHECK(h, K.fused_cfl(p, in, h->parts, h->ctrl, s, tm));
-      h->nparts = ppk::fused_cfl_parts(p);
-    }
-    HIP_CHECK(h, K.set_dt(h->ctrl, h->parts, h->nparts, dt, mode, h->p.cfl, s));
-    if (march) {  // the single-pass step
-      HIP_CHECK(h, (p.dim == 3 ? K.march_godunov : K.march2d_godunov)(p, in, out, h->parts, h->ctrl,
-                                                                      cfl ? 1 : 0, s, tm));
-      if (cfl) h->nparts = (int)ppk::march_blocks(p);
-    } else {
-      HIP_CHECK(h, K.fused_godunov(p, in, out, h->fw, h->parts, h->ctrl, cfl ? 1 : 0, s, tm));
-      if (cfl) h->nparts = ppk::fused_cfl_parts(p);
-    }
-    h->cfl_valid = cfl;
-  } else {
+  if (!h->fused) {
+    HIP_CHECK(h, K.begin(h->ctrl, check_finished, s));
+    HIP_CHECK(h, K.boundaries(p, in, nullptr, h->ctrl, s, tm));
     const int nparts = ppk::cfl_blocks(p);
     HIP_CHECK(h, K.prim_dt(p, in, h->Q, h->parts, h->ctrl, cfl ? 1 : 0, s, tm));
     HIP_CHECK(h, K.set_dt(h->ctrl, h->parts, nparts, dt, mode, h->p.cfl, s));
     HIP_CHECK(h, K.godunov(p, in, out, h->Q, h->w, h->ctrl, s, tm));
+    HIP_CHECK(h, K.end(h->ctrl, s));
+    h->mirrored = false;
+    return PPK_OK;
   }
-  HIP_CHECK(h, K.end(h->ctrl, s));
+  // the single-pass step writes only the interior of its output: the ghost fill gives the
+  // output the filled input's ghosts (the reference's U2 = U copy) in the same pass
+  const bool march = p.march > 0 && !h->fw.sur;
+  // the previous fused step left the CFL maxima of its output (= in) in parts; the prologue
+  // takes dt from them unless they are missing or too many for one block
+  const bool fresh = cfl && !h->cfl_valid;
+  const bool later = fresh || (cfl && h->nparts > ppk::kPrologueParts);
+  HIP_CHECK(h, K.prologue(p, in, march ? out : nullptr, h->ctrl, h->parts, h->nparts, dt,
+                          later ? ppk::SETDT_LATER : mode, h->p.cfl, check_finished, s, tm));
+  if (fresh) {
+    HIP_CHECK(h, K.fused_cfl(p, in, h->parts, h->ctrl, s, tm));
+    h->nparts = ppk::fused_cfl_parts(p);
+  }
+  if (later) HIP_CHECK(h, K.set_dt(h->ctrl, h->parts, h->nparts, dt, mode, h->p.cfl, s));
+  if (march) {
+    HIP_CHECK(h, (p.dim == 3 ? K.march_godunov : K.march2d_godunov)(
+                     p, in, out, h->parts, h->ctrl, h->mirror, cfl ? 1 : 0, s, tm));
+    if (cfl) h->nparts = (int)ppk::march_blocks(p);
+  } else {
+    HIP_CHECK(h, K.fused_godunov(p, in, out, h->fw, h->parts, h->ctrl, h->mirror, cfl ? 1 : 0, s,
+                                 tm));
+    if (cfl) h->nparts = ppk::fused_cfl_parts(p);
+  }
+  h->cfl_valid = cfl;
   return PPK_OK;
 }
 
@@ -410,11 +438,13 @@ int ppk_mhd_create(const ppk_mhd_params *params, ppk_mhd_t **handle) {
   // them (they are allocated when the surrogate or a face dump first asks for them)
   if (ok && h->fused && h->dp.march == 0) ok = alloc_records(h);
   if (!ok) return bail(PPK_ERR_OUT_OF_MEMORY, "device allocation failed");
-  if (hipHostMalloc((void **)&h->ctrl_host, sizeof(double) * (ppk::CTRL_SLOTS + 1)) != hipSuccess)
+  if (hipHostMalloc((void **)&h->ctrl_host, sizeof(double) * (2 * ppk::CTRL_SLOTS + 8)) !=
+      hipSuccess)
     return bail(PPK_ERR_OUT_OF_MEMORY, "pinned host allocation failed");
   if (hipMemsetAsync(h->U[0], 0, 8 * n * sizeof(double), h->stream) != hipSuccess ||
       hipMemsetAsync(h->U[1], 0, 8 * n * sizeof(double), h->stream) != hipSuccess)
     return bail(PPK_ERR_HIP, "hipMemsetAsync failed");
+  h->mirror = h->ctrl_host + ppk::CTRL_SLOTS + 8;
   std::fill(h->ctrl_host, h->ctrl_host + ppk::CTRL_SLOTS, 0.0);
   // SolverBase::read_config: t = tCurrent (0), dt = tEnd (src/shared/SolverBase.cpp:119-121)
   h->ctrl_host[ppk::CTRL_T] = 0.0;
@@ -558,6 +588,7 @@ int ppk_mhd_compute_dt(ppk_mhd_t *h, double *dt) {
   if (h->fused) h->nparts = nparts;
   HIP_CHECK(h, h->K->set_dt(h->ctrl, h->parts, nparts, 0.0,
                             ppk::SETDT_REDUCE_ONLY, h->p.cfl, h->stream));
+  h->mirrored = false;
   int rc = read_ctrl(h);
   if (rc != PPK_OK) return rc;
   *dt = h->p.cfl / h->ctrl_host[ppk::CTRL_INVDT];
@@ -585,6 +616,7 @@ int ppk_mhd_dump_faces(ppk_mhd_t *h, ppk_faceset_t *set, int stride, int phase,
   HIP_CHECK(h, h->K->fused_cfl(h->dp, h->cur(), h->parts, h->ctrl, h->stream, h->tm()));
   HIP_CHECK(h, h->K->set_dt(h->ctrl, h->parts, ppk::fused_cfl_parts(h->dp), 0.0,
                             ppk::SETDT_CFL, h->p.cfl, h->stream));
+  h->mirrored = false;
   HIP_CHECK(h, h->K->fused_half(h->dp, h->cur(), h->fw.rec, h->ctrl, h->stream));
   HIP_CHECK(h, h->K->surrogate_dump(h->dp, h->fw.rec, h->ctrl, set->X + set->n * ppk::kMlpIn,
                                     set->T + set->n * ppk::kMlpOut, stride, phase, h->stream));

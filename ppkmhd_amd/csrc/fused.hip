@@ -156,11 +156,13 @@ __global__ void __launch_bounds__(kCflBlock) k_update(const double *__restrict__
                                                       const R *__restrict__ flux,
                                                       const double *__restrict__ emf,
                                                       double *__restrict__ parts, DevParams p,
-                                                      Brick bk, const double *ctrl, int fold) {
+                                                      Brick bk, double *ctrl, double *host,
+                                                      int fold) {
   if (!active(ctrl)) return;
   __shared__ double red[kCflBlock / 64];
   const double dt = ctrl[CTRL_DT];
   const double dtdx = dt / p.dx, dtdy = dt / p.dy, dtdz = p.dim == 3 ? dt / p.dz : 0.0;
+  if (blockIdx.x == 0 && threadIdx.x == 0) step_end(ctrl, host);
   int i, j, k;
   double best = 0.0;
   if (brick_cell(bk, xcd_remap(blockIdx.x, gridDim.x), threadIdx.x, i, j, k))
@@ -242,7 +244,7 @@ void launch_half3(const DevParams &p, const double *Uin, R *rec, const double *c
 // rec and flux hold R, emf holds double
 template <class R>
 hipError_t godunov_impl(const DevParams &p, const double *Uin, double *Uout, R *rec, R *flux,
-                        double *emf, double *parts, const double *ctrl, int fold_cfl,
+                        double *emf, double *parts, double *ctrl, double *host, int fold_cfl,
                         const SurrogateCfg *sur, hipStream_t s, StageTimer *tm) {
   const Brick bk = sub_bricks(p);
   const dim3 g((unsigned)bk.count()), b(kRiemannBlock);
@@ -275,7 +277,8 @@ hipError_t godunov_impl(const DevParams &p, const double *Uin, double *Uout, R *
   }
   PPK_TIMED(tm, ST_FUSED_UPDATE,
             hipLaunchKernelGGL((k_update<R>), dim3(fused_cfl_parts(p)), dim3(kCflBlock), 0, s,
-                               Uin, Uout, flux, emf, parts, p, padded_bricks(p), ctrl, fold_cfl));
+                               Uin, Uout, flux, emf, parts, p, padded_bricks(p), ctrl, host,
+                               fold_cfl));
   return hipGetLastError();
 }
 
@@ -285,16 +288,16 @@ hipError_t godunov_impl(const DevParams &p, const double *Uin, double *Uout, R *
 // launchers
 // -------------------------------------------------------------------------------------------
 hipError_t fused_godunov(const DevParams &p, const double *Uin, double *Uout, FusedScratch &w,
-                         double *parts, const double *ctrl, int fold_cfl, hipStream_t s,
+                         double *parts, double *ctrl, double *host, int fold_cfl, hipStream_t s,
                          StageTimer *tm) {
   using namespace fusedk;
   if (p.bulk32)
     return godunov_impl<float>(p, Uin, Uout, static_cast<float *>(w.rec),
                                static_cast<float *>(w.flux), static_cast<double *>(w.emf), parts,
-                               ctrl, fold_cfl, w.sur, s, tm);
+                               ctrl, host, fold_cfl, w.sur, s, tm);
   return godunov_impl<double>(p, Uin, Uout, static_cast<double *>(w.rec),
                               static_cast<double *>(w.flux), static_cast<double *>(w.emf), parts,
-                              ctrl, fold_cfl, w.sur, s, tm);
+                              ctrl, host, fold_cfl, w.sur, s, tm);
 }
 
 template <class R>

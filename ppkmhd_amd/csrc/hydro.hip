@@ -147,49 +147,29 @@ __device__ __forceinline__ double inv_dt_cell(const HSt<NV> &u, const G3 &g, con
   return inv_dt_prim<GR>(q, c, g, h);
 }
 
-// ---- ghost fill, one direction, both faces (MakeBoundariesFunctor2D/3D,
+// ---- ghost fill of every face, edge and corner in one pass (ghost_shell_element: the values of
+// the reference's x, y, z passes, MakeBoundariesFunctor2D/3D,
 // src/shared/BoundariesFunctors.h:18-531): Dirichlet reflects and flips the normal velocity,
-// Neumann copies the first interior cell, periodic wraps
+// Neumann copies the first interior cell, periodic wraps.  One launch where three direction
+// passes took 37 us (256 x 192 x 128).
 template <int NV>
 __global__ void __launch_bounds__(kBlock) k_hbnd(double *__restrict__ U, double *__restrict__ C,
-                                                 HydroDev h, int dir, const double *ctrl) {
+                                                 HydroDev h, const double *ctrl) {
   if (!active(ctrl)) return;
-  const int gw = h.gw;
-  const int n = dir == 0 ? h.nx : (dir == 1 ? h.ny : h.nz);
-  const int s1 = dir == 0 ? h.jsize : h.isize;
-  const int s2 = dir == 2 ? h.jsize : h.ksize;
-  const long long total = 2LL * gw * s1 * s2;
+  const long long total = ghost_shell_cells(h);
   for (long long t = blockIdx.x * (long long)blockDim.x + threadIdx.x; t < total;
-       t += (long long)gridDim.x * blockDim.x) {
-    const int g = (int)(t % gw);
-    long long r = t / gw;
-    const int t1 = (int)(r % s1);
-    r /= s1;
-    const int t2 = (int)(r % s2);
-    const int upper = (int)(r / s2);
-    const int bc = h.bc[2 * dir + upper];
-    const int c = upper ? g + n + gw : g;
-    int c0;
-    if (bc == PPK_BC_DIRICHLET)
-      c0 = upper ? 2 * n + 2 * gw - 1 - c : 2 * gw - 1 - c;
-    else if (bc == PPK_BC_NEUMANN)
-      c0 = upper ? n + gw - 1 : gw;
-    else
-      c0 = upper ? c - n : n + c;
-    int i, j, k, i0, j0, k0;
-    if (dir == 0) { i = c; j = t1; k = t2; i0 = c0; j0 = j; k0 = k; }
-    else if (dir == 1) { i = t1; j = c; k = t2; i0 = i; j0 = c0; k0 = k; }
-    else { i = t1; j = t2; k = c; i0 = i; j0 = j; k0 = c0; }
-    const long long dst = ((long long)k * h.jsize + j) * h.isize + i;
-    const long long src = ((long long)k0 * h.jsize + j0) * h.isize + i0;
-#pragma unroll
-    for (int v = 0; v < NV; ++v) {
-      const double sign = (bc == PPK_BC_DIRICHLET && v == IU + dir) ? -1.0 : 1.0;
-      const double x = U[src + v * h.vstride] * sign;
-      U[dst + v * h.vstride] = x;
-      if (C) C[dst + v * h.vstride] = x;
-    }
-  }
+       t += (long long)gridDim.x * blockDim.x)
+    ghost_shell_element<NV>(U, h, t, C);
+}
+template <int NV>
+__global__ void __launch_bounds__(kBlock) k_hprologue(double *__restrict__ U,
+                                                      double *__restrict__ C, HydroDev h,
+                                                      double *ctrl,
+                                                      const double *__restrict__ parts,
+                                                      int nparts, double fixed_dt, int mode,
+                                                      double cfl, int check_finished) {
+  __shared__ double red[kBlock / 64];
+  step_prologue<NV>(U, C, h, ctrl, parts, nparts, fixed_dt, mode, cfl, check_finished, red);
 }
 
 // ---- primitives of every cell (ConvertToPrimitivesFunctor, SolverHydroMuscl.h) and the CFL
@@ -347,7 +327,8 @@ template <int NV, int RS, int MINW, int GR>
 __global__ void __launch_bounds__(kWaves2 * 64, MINW) k_hfused2d(const double *__restrict__ Uin,
                                                            double *__restrict__ Uout, HydroDev h,
                                                            double *__restrict__ parts,
-                                                           const double *ctrl, int fold_cfl) {
+                                                           double *ctrl, double *host,
+                                                           int fold_cfl) {
   if (!active(ctrl)) return;
   const int lane = threadIdx.x & 63;
   const int wave = blockIdx.x * kWaves2 + (threadIdx.x >> 6);
@@ -355,6 +336,7 @@ __global__ void __launch_bounds__(kWaves2 * 64, MINW) k_hfused2d(const double *_
   const int H = h.strip_rows;
   const int nsy = (h.ny + H - 1) / H;
   if (wave >= nsx * nsy) return;  // whole waves only
+  if (wave == 0 && lane == 0) step_end(ctrl, host);
   const int sx = wave % nsx, sy = wave / nsx;
   const int i = h.gw + sx * kHydroCols + lane - 2;
   const int ic = i < h.isize ? i : h.isize - 1;  // lanes past the box: clamped, never output
@@ -461,12 +443,14 @@ template <int NV, int RS, int MINW, int GR>
 __global__ void __launch_bounds__(kW3 * 64, MINW) k_hfused3d(const double *__restrict__ Uin,
                                                        double *__restrict__ Uout, HydroDev h,
                                                        double *__restrict__ parts,
-                                                       const double *ctrl, int fold_cfl) {
+                                                       double *ctrl, double *host,
+                                                       int fold_cfl) {
   constexpr int RW = kHydroRowW3, NR = kHydroBlockRows3;
   __shared__ double sQ[2][NV][NR][RW];  // Q of plane s (parity s & 1), later the y fluxes
   __shared__ double sT[NV][NR][RW];     // upper y-face states of plane s
   __shared__ double red[kW3];
   if (!active(ctrl)) return;
+  if (blockIdx.x == 0 && threadIdx.x == 0) step_end(ctrl, host);
   const int lane = threadIdx.x % RW;  // column within the row
   const int ly = threadIdx.x / RW;    // row of the block
   const int nsx = (h.nx + kHydroCols3 - 1) / kHydroCols3;
@@ -631,15 +615,25 @@ int fused3d_blocks(const HydroDev &h) {
 // -------------------------------------------------------------------------------------------
 hipError_t hydro_boundaries(const HydroDev &h, double *U, double *copy, const double *ctrl,
                             hipStream_t s) {
-  for (int dir = 0; dir < h.dim; ++dir) {
-    const int s1 = dir == 0 ? h.jsize : h.isize;
-    const int s2 = dir == 2 ? h.jsize : h.ksize;
-    const long long n = 2LL * h.gw * s1 * s2;
-    if (h.dim == 3)
-      hipLaunchKernelGGL(k_hbnd<5>, dim3(grid_for(n)), dim3(kBlock), 0, s, U, copy, h, dir, ctrl);
-    else
-      hipLaunchKernelGGL(k_hbnd<4>, dim3(grid_for(n)), dim3(kBlock), 0, s, U, copy, h, dir, ctrl);
-  }
+  const dim3 g(grid_for(ghost_shell_cells(h))), b(kBlock);
+  if (h.dim == 3)
+    hipLaunchKernelGGL(k_hbnd<5>, g, b, 0, s, U, copy, h, ctrl);
+  else
+    hipLaunchKernelGGL(k_hbnd<4>, g, b, 0, s, U, copy, h, ctrl);
+  return hipGetLastError();
+}
+
+hipError_t hydro_prologue(const HydroDev &h, double *U, double *copy, double *ctrl,
+                          const double *parts, int nparts, double fixed_dt, int mode, double cfl,
+                          int check_finished, hipStream_t s) {
+  static_assert(kBlock == 256, "step_prologue is written for 256 threads");
+  const dim3 g(prologue_blocks(ghost_shell_cells(h))), b(kBlock);
+  if (h.dim == 3)
+    hipLaunchKernelGGL(k_hprologue<5>, g, b, 0, s, U, copy, h, ctrl, parts, nparts, fixed_dt, mode,
+                       cfl, check_finished);
+  else
+    hipLaunchKernelGGL(k_hprologue<4>, g, b, 0, s, U, copy, h, ctrl, parts, nparts, fixed_dt, mode,
+                       cfl, check_finished);
   return hipGetLastError();
 }
 
@@ -700,42 +694,42 @@ int hydro_fused_parts(const HydroDev &h) {
 
 template <int RS, int GR>
 void launch_fused_gr(const HydroDev &h, const double *Uin, double *Uout, double *parts,
-                     const double *ctrl, int fold_cfl, hipStream_t s) {
+                     double *ctrl, double *host, int fold_cfl, hipStream_t s) {
   if (h.dim == 3) {
     if constexpr (RS != PPK_RIEMANN_HLL) {  // no 3D HLL (refused at create)
       const dim3 g(fused3d_blocks(h)), b(kW3 * 64);
       hipLaunchKernelGGL((k_hfused3d<5, RS, 1, GR>), g, b, 0, s, Uin, Uout, h, parts, ctrl,
-                         fold_cfl);
+                         host, fold_cfl);
     }
   } else {
     const int waves = fused2d_waves(h);
     const dim3 g((waves + kWaves2 - 1) / kWaves2), b(kWaves2 * 64);
     hipLaunchKernelGGL((k_hfused2d<4, RS, 1, GR>), g, b, 0, s, Uin, Uout, h, parts, ctrl,
-                       fold_cfl);
+                       host, fold_cfl);
   }
 }
 
 // the fused kernels with or without the gravity terms
 template <int RS>
 void launch_fused(const HydroDev &h, const double *Uin, double *Uout, double *parts,
-                  const double *ctrl, int fold_cfl, hipStream_t s) {
+                  double *ctrl, double *host, int fold_cfl, hipStream_t s) {
   if (h.grav)
-    launch_fused_gr<RS, 1>(h, Uin, Uout, parts, ctrl, fold_cfl, s);
+    launch_fused_gr<RS, 1>(h, Uin, Uout, parts, ctrl, host, fold_cfl, s);
   else
-    launch_fused_gr<RS, 0>(h, Uin, Uout, parts, ctrl, fold_cfl, s);
+    launch_fused_gr<RS, 0>(h, Uin, Uout, parts, ctrl, host, fold_cfl, s);
 }
 
 hipError_t hydro_fused(const HydroDev &h, const double *Uin, double *Uout, double *parts,
-                       const double *ctrl, int fold_cfl, hipStream_t s) {
+                       double *ctrl, double *host, int fold_cfl, hipStream_t s) {
   switch (h.P.riemann) {  // the solver as a compile-time constant of the kernel
     case PPK_RIEMANN_APPROX:
-      launch_fused<PPK_RIEMANN_APPROX>(h, Uin, Uout, parts, ctrl, fold_cfl, s);
+      launch_fused<PPK_RIEMANN_APPROX>(h, Uin, Uout, parts, ctrl, host, fold_cfl, s);
       break;
-    case PPK_RIEMANN_HLL: launch_fused<PPK_RIEMANN_HLL>(h, Uin, Uout, parts, ctrl, fold_cfl, s); break;
+    case PPK_RIEMANN_HLL: launch_fused<PPK_RIEMANN_HLL>(h, Uin, Uout, parts, ctrl, host, fold_cfl, s); break;
     case PPK_RIEMANN_HLLC:
-      launch_fused<PPK_RIEMANN_HLLC>(h, Uin, Uout, parts, ctrl, fold_cfl, s);
+      launch_fused<PPK_RIEMANN_HLLC>(h, Uin, Uout, parts, ctrl, host, fold_cfl, s);
       break;
-    default: launch_fused<PPK_RIEMANN_LLF>(h, Uin, Uout, parts, ctrl, fold_cfl, s); break;
+    default: launch_fused<PPK_RIEMANN_LLF>(h, Uin, Uout, parts, ctrl, host, fold_cfl, s); break;
   }
   return hipGetLastError();
 }

@@ -26,11 +26,13 @@ const char *const kHydroStageNames[HS_COUNT] = {"boundaries", "primitives_dt", "
                                                 "update", "fused", "control"};
 static_assert(HS_COUNT <= ST_COUNT, "the event timer holds ST_COUNT stages");
 
-const HydroTable kHydroFast = {fast::hydro_boundaries,    fast::hydro_prim_dt,
+const HydroTable kHydroFast = {fast::hydro_boundaries,    fast::hydro_prologue,
+                               fast::hydro_prim_dt,
                                fast::hydro_prim_parts,    fast::hydro_staged_fluxes,
                                fast::hydro_staged_update, fast::hydro_fused,
                                fast::hydro_fused_parts};
-const HydroTable kHydroStrict = {strict::hydro_boundaries,    strict::hydro_prim_dt,
+const HydroTable kHydroStrict = {strict::hydro_boundaries,    strict::hydro_prologue,
+                                 strict::hydro_prim_dt,
                                  strict::hydro_prim_parts,    strict::hydro_staged_fluxes,
                                  strict::hydro_staged_update, strict::hydro_fused,
                                  strict::hydro_fused_parts};
@@ -445,7 +447,10 @@ struct ppk_hydro_solver {
   double *F = nullptr;  // staged form: dim x nv flux planes
   double *G = nullptr;  // gravity: dim planes of the per-cell field
   double *ctrl = nullptr;
-  double *ctrl_host = nullptr;
+  double *ctrl_host = nullptr;  // pinned: the control block as the host last read or wrote it,
+                                // then the mirror
+  double *mirror = nullptr;     // what the fused step's kernel wrote of it (as in ppk_mhd_solver)
+  bool mirrored = false;
   double *parts = nullptr;
   ppk::EventTimer *timer = nullptr;
   bool fused = false;
@@ -480,17 +485,28 @@ int hfail(ppk_hydro_t *h, int code, const std::string &msg) {
       return hfail((h), PPK_ERR_HIP, std::string(#expr) + ": " + hipGetErrorString(_e));  \
   } while (0)
 
+constexpr int kMirrored[4] = {ppk::CTRL_T, ppk::CTRL_DT, ppk::CTRL_INVDT, ppk::CTRL_ITER};
+
 int hwrite_ctrl(ppk_hydro_t *h) {
   HHIP(h, hipMemcpyAsync(h->ctrl, h->ctrl_host, sizeof(double) * ppk::CTRL_SLOTS,
                          hipMemcpyHostToDevice, h->stream));
   HHIP(h, hipStreamSynchronize(h->stream));
+  for (int i : kMirrored) h->mirror[i] = h->ctrl_host[i];
+  h->mirrored = true;
   return PPK_OK;
 }
 
 int hread_ctrl(ppk_hydro_t *h) {
+  if (h->mirrored) {
+    HHIP(h, hipStreamSynchronize(h->stream));
+    for (int i : kMirrored) h->ctrl_host[i] = h->mirror[i];
+    return PPK_OK;
+  }
   HHIP(h, hipMemcpyAsync(h->ctrl_host, h->ctrl, sizeof(double) * ppk::CTRL_SLOTS,
                          hipMemcpyDeviceToHost, h->stream));
   HHIP(h, hipStreamSynchronize(h->stream));
+  for (int i : kMirrored) h->mirror[i] = h->ctrl_host[i];
+  h->mirrored = true;
   return PPK_OK;
 }
 
@@ -514,19 +530,25 @@ int hlaunch_step(ppk_hydro_t *h, double dt, int dt_mode, int check_finished) {
   const bool cfl = dt_mode == PPK_DT_CFL;
   const int mode = cfl ? ppk::SETDT_CFL : ppk::SETDT_FIXED;
   ppk::StageTimer *tm = h->tm();
-  HHIP(h, K.begin(h->ctrl, check_finished, s));
   if (h->fused) {
-    PPK_TIMED(tm, ppk::HS_BOUNDARIES, HHIP(h, H.boundaries(d, in, out, h->ctrl, s)));
+    const bool fresh = cfl && !h->cfl_valid;
     int nparts = H.fused_parts(d);
-    if (cfl && !h->cfl_valid) {
+    const bool later = fresh || (cfl && nparts > ppk::kPrologueParts);
+    PPK_TIMED(tm, ppk::HS_BOUNDARIES,
+              HHIP(h, H.prologue(d, in, out, h->ctrl, h->parts, nparts, dt,
+                                 later ? ppk::SETDT_LATER : mode, h->p.cfl, check_finished, s)));
+    if (fresh) {
       PPK_TIMED(tm, ppk::HS_PRIM_DT, HHIP(h, H.prim_dt(d, in, nullptr, h->parts, h->ctrl, 1, s)));
       nparts = H.prim_parts(d);
     }
-    PPK_TIMED(tm, ppk::HS_CONTROL,
-              HHIP(h, K.set_dt(h->ctrl, h->parts, nparts, dt, mode, h->p.cfl, s)));
-    PPK_TIMED(tm, ppk::HS_FUSED, HHIP(h, H.fused(d, in, out, h->parts, h->ctrl, cfl ? 1 : 0, s)));
+    if (later)
+      PPK_TIMED(tm, ppk::HS_CONTROL,
+                HHIP(h, K.set_dt(h->ctrl, h->parts, nparts, dt, mode, h->p.cfl, s)));
+    PPK_TIMED(tm, ppk::HS_FUSED,
+              HHIP(h, H.fused(d, in, out, h->parts, h->ctrl, h->mirror, cfl ? 1 : 0, s)));
     h->cfl_valid = cfl;
   } else {
+    HHIP(h, K.begin(h->ctrl, check_finished, s));
     PPK_TIMED(tm, ppk::HS_BOUNDARIES, HHIP(h, H.boundaries(d, in, nullptr, h->ctrl, s)));
     PPK_TIMED(tm, ppk::HS_PRIM_DT,
               HHIP(h, H.prim_dt(d, in, h->Q, h->parts, h->ctrl, cfl ? 1 : 0, s)));
@@ -535,8 +557,9 @@ int hlaunch_step(ppk_hydro_t *h, double dt, int dt_mode, int check_finished) {
     HHIP(h, hipMemcpyAsync(out, in, h->state_bytes(), hipMemcpyDeviceToDevice, s));
     PPK_TIMED(tm, ppk::HS_FLUXES, HHIP(h, H.staged_fluxes(d, h->Q, h->F, h->ctrl, s)));
     PPK_TIMED(tm, ppk::HS_UPDATE, HHIP(h, H.staged_update(d, h->F, out, h->ctrl, s)));
+    HHIP(h, K.end(h->ctrl, s));
+    h->mirrored = false;
   }
-  HHIP(h, K.end(h->ctrl, s));
   return PPK_OK;
 }
 
@@ -627,11 +650,12 @@ int ppk_hydro_create(const ppk_mhd_params *params, ppk_hydro_t **handle) {
   if (h->G && hipMemsetAsync(h->G, 0, (size_t)params->dim * h->cells() * sizeof(double),
                              h->stream) != hipSuccess)
     return bail(PPK_ERR_HIP, "hipMemsetAsync failed");
-  if (hipHostMalloc((void **)&h->ctrl_host, sizeof(double) * ppk::CTRL_SLOTS) != hipSuccess)
+  if (hipHostMalloc((void **)&h->ctrl_host, sizeof(double) * 2 * ppk::CTRL_SLOTS) != hipSuccess)
     return bail(PPK_ERR_OUT_OF_MEMORY, "pinned host allocation failed");
   if (hipMemsetAsync(h->U[0], 0, nvals * sizeof(double), h->stream) != hipSuccess ||
       hipMemsetAsync(h->U[1], 0, nvals * sizeof(double), h->stream) != hipSuccess)
     return bail(PPK_ERR_HIP, "hipMemsetAsync failed");
+  h->mirror = h->ctrl_host + ppk::CTRL_SLOTS;
   std::fill(h->ctrl_host, h->ctrl_host + ppk::CTRL_SLOTS, 0.0);
   h->ctrl_host[ppk::CTRL_DT] = params->tEnd;
   h->ctrl_host[ppk::CTRL_TEND] = params->tEnd;
@@ -735,6 +759,7 @@ int ppk_hydro_compute_dt(ppk_hydro_t *h, double *dt) {
   HHIP(h, h->K->set_dt(h->ctrl, h->parts, h->H->prim_parts(h->hd), 0.0,
                        ppk::SETDT_REDUCE_ONLY, h->p.cfl, h->stream));
   h->cfl_valid = false;
+  h->mirrored = false;
   int rc = hread_ctrl(h);
   if (rc != PPK_OK) return rc;
   *dt = h->p.cfl / h->ctrl_host[ppk::CTRL_INVDT];

@@ -43,10 +43,14 @@ constexpr int kHydroRows3 = kHydroBlockRows3 - 4;
 
 #define PPK_DECLARE_HYDRO(NS)                                                                    \
   namespace NS {                                                                                 \
-  /* ghost fill of U (x, then y, then z); with copy != nullptr every ghost value is also        \
+  /* ghost fill of U in one pass (the values of x, then y, then z passes); with copy != nullptr every ghost value is also        \
      written there (the next state's ghosts = this state's, as the reference's deep copy) */    \
   hipError_t hydro_boundaries(const HydroDev &h, double *U, double *copy, const double *ctrl,    \
                               hipStream_t s);                                                    \
+  /* the finished test, the ghost fill and dt in one launch (staged_prologue) */                 \
+  hipError_t hydro_prologue(const HydroDev &h, double *U, double *copy, double *ctrl,            \
+                            const double *parts, int nparts, double fixed_dt, int mode,          \
+                            double cfl, int check_finished, hipStream_t s);                      \
   /* primitives of every cell into Q (staged form) and per-block CFL maxima of the interior */   \
   hipError_t hydro_prim_dt(const HydroDev &h, const double *U, double *Q, double *parts,         \
                            const double *ctrl, int do_dt, hipStream_t s);                        \
@@ -58,9 +62,9 @@ constexpr int kHydroRows3 = kHydroBlockRows3 - 4;
   hipError_t hydro_staged_update(const HydroDev &h, const double *F, double *Uout,               \
                                  const double *ctrl, hipStream_t s);                             \
   /* fused form: one marching kernel from Uin to the interior of Uout; with fold_cfl the        \
-     per-wave / per-block CFL maxima of the new state go to parts */                             \
+     per-wave / per-block CFL maxima of the new state go to parts; ends the step (step_end) */   \
   hipError_t hydro_fused(const HydroDev &h, const double *Uin, double *Uout, double *parts,      \
-                         const double *ctrl, int fold_cfl, hipStream_t s);                       \
+                         double *ctrl, double *host, int fold_cfl, hipStream_t s);               \
   int hydro_fused_parts(const HydroDev &h);                                                      \
   }
 
@@ -69,6 +73,7 @@ PPK_DECLARE_HYDRO(strict)
 
 struct HydroTable {
   decltype(&fast::hydro_boundaries) boundaries;
+  decltype(&fast::hydro_prologue) prologue;
   decltype(&fast::hydro_prim_dt) prim_dt;
   decltype(&fast::hydro_prim_parts) prim_parts;
   decltype(&fast::hydro_staged_fluxes) staged_fluxes;

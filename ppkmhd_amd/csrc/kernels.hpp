@@ -89,8 +89,12 @@ struct FusedScratch {
   const SurrogateCfg *sur = nullptr;  // surrogate face solves when set
 };
 
-// dt modes of the set_dt kernel
-enum { SETDT_FIXED = 0, SETDT_CFL = 1, SETDT_REDUCE_ONLY = 2 };
+// dt modes of the set_dt kernel; SETDT_LATER: a prologue that leaves dt to a later set_dt
+enum { SETDT_FIXED = 0, SETDT_CFL = 1, SETDT_REDUCE_ONLY = 2, SETDT_LATER = 3 };
+// CFL partials that the prologue's one block of 256 threads reduces itself; more of them go to
+// set_dt (1024 threads).  8192 take four rounds of eight loads per thread, about 3 us, which
+// the ghost fill beside it covers.
+constexpr int kPrologueParts = 8192;
 
 // The CFL maximum is produced as per-block partial maxima (no same-address atomics): each
 // block of a producer kernel writes its slot, set_dt reduces as many slots as the producer had
@@ -223,6 +227,11 @@ struct BatchMember {
   /* ghost fill of U; copy (may be null) receives the same ghost values */                     \
   hipError_t staged_boundaries(const DevParams &p, double *U, double *copy, const double *ctrl,  \
                                hipStream_t s, StageTimer *tm);                                   \
+  /* the finished test, the ghost fill (copy as above) and dt in one launch; nparts at most      \
+     kPrologueParts unless mode is SETDT_FIXED or SETDT_LATER */                                \
+  hipError_t staged_prologue(const DevParams &p, double *U, double *copy, double *ctrl,          \
+                             const double *parts, int nparts, double fixed_dt, int mode,         \
+                             double cfl, int check_finished, hipStream_t s, StageTimer *tm);     \
   hipError_t staged_prim_dt(const DevParams &p, const double *U, double *Q, double *parts,       \
                             const double *ctrl, int do_dt, hipStream_t s, StageTimer *tm);       \
   hipError_t staged_begin(double *ctrl, int check_finished, hipStream_t s);                      \
@@ -232,9 +241,10 @@ struct BatchMember {
   hipError_t staged_godunov(const DevParams &p, const double *Uin, double *Uout,                 \
                             const double *Q, StagedScratch &w, const double *ctrl,               \
                             hipStream_t s, StageTimer *tm);                                      \
+  /* the fused steps: their last kernel ends the step (step_end, `host` its pinned copy) */      \
   hipError_t fused_godunov(const DevParams &p, const double *Uin, double *Uout,                  \
-                           FusedScratch &w, double *parts, const double *ctrl, int fold_cfl,     \
-                           hipStream_t s, StageTimer *tm);                                       \
+                           FusedScratch &w, double *parts, double *ctrl, double *host,           \
+                           int fold_cfl, hipStream_t s, StageTimer *tm);                         \
   hipError_t fused_cfl(const DevParams &p, const double *U, double *parts, const double *ctrl,   \
                        hipStream_t s, StageTimer *tm);                                           \
   hipError_t fused_half(const DevParams &p, const double *U, void *rec, const double *ctrl,      \
@@ -249,10 +259,12 @@ struct BatchMember {
   /* single-pass 3D step (p.march > 0): the interior of Uout (its ghosts come from the ghost   \
      fill's copy target); CFL partials, one per block, when fold_cfl */                         \
   hipError_t march_godunov(const DevParams &p, const double *Uin, double *Uout, double *parts,   \
-                           const double *ctrl, int fold_cfl, hipStream_t s, StageTimer *tm);    \
+                           double *ctrl, double *host, int fold_cfl, hipStream_t s,              \
+                           StageTimer *tm);                                                      \
   /* the same in 2D: CFL partials, one per wave */                                             \
   hipError_t march2d_godunov(const DevParams &p, const double *Uin, double *Uout, double *parts, \
-                             const double *ctrl, int fold_cfl, hipStream_t s, StageTimer *tm);  \
+                             double *ctrl, double *host, int fold_cfl, hipStream_t s,            \
+                             StageTimer *tm);                                                    \
   /* batched ensemble: counts of blocks per stage for one member, then the batched step */      \
   void batch_block_counts(const DevParams &p, int tile, long long counts[BS_COUNT]);            \
   hipError_t batch_step(const BatchMember *members, int nmembers, int dim, int bulk32, int tile, \
@@ -265,6 +277,7 @@ PPK_DECLARE_KERNELS(strict)
 // entry-point table of one arithmetic variant
 struct KernelTable {
   decltype(&fast::staged_boundaries) boundaries;
+  decltype(&fast::staged_prologue) prologue;
   decltype(&fast::staged_prim_dt) prim_dt;
   decltype(&fast::staged_begin) begin;
   decltype(&fast::staged_set_dt) set_dt;
@@ -295,7 +308,8 @@ extern const KernelTable kStrict;
 // receives the same ghost values, the single-pass step's output whose ghosts are the
 // reference's U2 = U copy of the filled input).
 // source coordinate of c in [0, n + 2 gw) along one direction; flip: a Dirichlet face mapped it
-PPK_HD int ghost_src(const DevParams &p, int d, int c, bool &flip) {
+template <class P>
+PPK_HD int ghost_src(const P &p, int d, int c, bool &flip) {
   const int gw = p.gw, n = d == 0 ? p.nx : (d == 1 ? p.ny : p.nz);
   flip = false;
   if (c >= gw && c < n + gw) return c;
@@ -310,36 +324,36 @@ PPK_HD int ghost_src(const DevParams &p, int d, int c, bool &flip) {
 }
 // ghost cells of the padded box: the 2 gw z planes (3D), then per interior plane the 2 gw y
 // rows, then per interior row the 2 gw x cells
-PPK_HD long long ghost_shell_cells(const DevParams &p) {
+template <class P>
+PPK_HD long long ghost_shell_cells(const P &p) {
   const long long gw2 = 2LL * p.gw, kin = p.dim == 3 ? p.nz : 1;
   return (p.dim == 3 ? gw2 * p.jsize * p.isize : 0) + kin * gw2 * p.isize + kin * p.ny * gw2;
 }
-PPK_HD void ghost_shell_element(double *__restrict__ U, const DevParams &p, long long t,
+template <int NV = 8, class P>
+PPK_HD void ghost_shell_element(double *__restrict__ U, const P &p, long long cell,
                                 double *__restrict__ copy) {
-  const int gw = p.gw;
-  const long long gw2 = 2LL * gw;
-  const long long nA = p.dim == 3 ? gw2 * p.jsize * p.isize : 0;
-  const long long nB = (p.dim == 3 ? p.nz : 1) * gw2 * p.isize;
-  const int koff = p.dim == 3 ? gw : 0;
+  // grids have at most 2^31 padded cells: 32-bit arithmetic
+  const unsigned t = (unsigned)cell, gw = (unsigned)p.gw, gw2 = 2 * gw;
+  const unsigned is = (unsigned)p.isize, js = (unsigned)p.jsize, ny = (unsigned)p.ny;
+  const unsigned nA = p.dim == 3 ? gw2 * js * is : 0u;
+  const unsigned nB = (p.dim == 3 ? (unsigned)p.nz : 1u) * gw2 * is;
+  const int koff = p.dim == 3 ? p.gw : 0;
   int i, j, k;
   if (t < nA) {
-    const int kk = (int)(t / ((long long)p.jsize * p.isize));
-    k = kk < gw ? kk : p.nz + kk;
-    j = (int)((t / p.isize) % p.jsize);
-    i = (int)(t % p.isize);
+    const unsigned row = t / is, kk = row / js;
+    k = (int)(kk < gw ? kk : (unsigned)p.nz + kk);
+    j = (int)(row - kk * js);
+    i = (int)(t - row * is);
   } else if (t < nA + nB) {
-    const long long u = t - nA;
-    k = (int)(u / (gw2 * p.isize)) + koff;
-    const int jj = (int)((u / p.isize) % gw2);
-    j = jj < gw ? jj : p.ny + jj;
-    i = (int)(u % p.isize);
+    const unsigned u = t - nA, row = u / is, kk = row / gw2, jj = row - kk * gw2;
+    k = (int)kk + koff;
+    j = (int)(jj < gw ? jj : ny + jj);
+    i = (int)(u - row * is);
   } else {
-    const long long u = t - nA - nB;
-    k = (int)(u / ((long long)p.ny * gw2)) + koff;
-    const long long r = u % ((long long)p.ny * gw2);
-    j = gw + (int)(r / gw2);
-    const int ii = (int)(r % gw2);
-    i = ii < gw ? ii : p.nx + ii;
+    const unsigned u = t - nA - nB, row = u / gw2, kk = row / ny, ii = u - row * gw2;
+    k = (int)kk + koff;
+    j = (int)(gw + (row - kk * ny));
+    i = (int)(ii < gw ? ii : (unsigned)p.nx + ii);
   }
   bool fx, fy, fz = false;
   const int i0 = ghost_src(p, 0, i, fx), j0 = ghost_src(p, 1, j, fy);
@@ -347,7 +361,7 @@ PPK_HD void ghost_shell_element(double *__restrict__ U, const DevParams &p, long
   const long long dst = ((long long)k * p.jsize + j) * p.isize + i;
   const long long src = ((long long)k0 * p.jsize + j0) * p.isize + i0;
 #pragma unroll
-  for (int v = 0; v < 8; ++v) {
+  for (int v = 0; v < NV; ++v) {  // NV < 8: the Euler solvers, no field
     const bool neg = ((v == IU || v == IA) && fx) != (((v == IV || v == IB) && fy) !=
                                                       ((v == IW || v == IC) && fz));
     const double x = U[src + v * p.vstride] * (neg ? -1.0 : 1.0);
@@ -367,6 +381,90 @@ __device__ __forceinline__ double block_max(double v, double *smem32) {
   for (int w = 1; w < nw; ++w) m = fmax(m, smem32[w]);
   __syncthreads();
   return m;
+}
+
+// ---- time-loop control, shared by the MHD and Euler steps ----------------------------------
+// SolverBase::finished() (src/shared/SolverBase.cpp:195-201), if the step was asked to check
+__device__ __forceinline__ bool step_wanted(const double *ctrl, int check_finished) {
+  return !check_finished || !(ctrl[CTRL_T] >= (ctrl[CTRL_TEND] - 1e-14) ||
+                              ctrl[CTRL_ITER] >= ctrl[CTRL_NSTEPMAX]);
+}
+// dt from the CFL partial maxima or the fixed value, clamped to tEnd - t,
+// src/muscl/SolverMHDMuscl.h:737 and src/shared/SolverBase.cpp:173-177.  One block of NT
+// threads; red: NT / 64 doubles of LDS.
+template <int NT>
+__device__ __forceinline__ void step_dt(double *ctrl, const double *__restrict__ parts,
+                                        int nparts, double fixed_dt, int mode, double cfl,
+                                        double *red) {
+  if (mode == SETDT_FIXED) {
+    // a fixed dt is clamped to tEnd like the CFL one (SolverBase.cpp:173-177), so a run of
+    // fixed steps stops exactly at tEnd
+    if (threadIdx.x == 0) {
+      double dt = fixed_dt;
+      if (ctrl[CTRL_T] + dt > ctrl[CTRL_TEND]) dt = ctrl[CTRL_TEND] - ctrl[CTRL_T];
+      ctrl[CTRL_DT] = dt;
+    }
+    return;
+  }
+  // eight independent loads in flight per thread: the partials can number ~10^5
+  double m[8] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+  int b = threadIdx.x;
+  for (; b + 7 * NT < nparts; b += 8 * NT) {
+#pragma unroll
+    for (int u = 0; u < 8; ++u) m[u] = fmax(m[u], parts[b + u * NT]);
+  }
+#pragma unroll
+  for (int u = 0; u < 8; ++u)
+    if (b + u * NT < nparts) m[u] = fmax(m[u], parts[b + u * NT]);
+#pragma unroll
+  for (int u = 1; u < 8; ++u) m[0] = fmax(m[0], m[u]);
+  const double mx = block_max(m[0], red);
+  if (threadIdx.x != 0) return;
+  ctrl[CTRL_INVDT] = mx;
+  if (mode == SETDT_CFL) {
+    double dt = cfl / mx;
+    if (ctrl[CTRL_T] + dt > ctrl[CTRL_TEND]) dt = ctrl[CTRL_TEND] - ctrl[CTRL_T];
+    ctrl[CTRL_DT] = dt;
+  }
+}
+// The prologue of a step in one launch: block 0 decides whether the step runs and sets its dt,
+// the others fill the ghosts (they decide for themselves from t and the iteration, which no
+// block of this launch writes).  Three launches (finished test, ghost fill, dt) took 14 us
+// between them on grids too small to hide them, this one 6.
+template <int NV, class P>
+__device__ __forceinline__ void step_prologue(double *__restrict__ U, double *__restrict__ copy,
+                                              const P &p, double *ctrl,
+                                              const double *__restrict__ parts, int nparts,
+                                              double fixed_dt, int mode, double cfl,
+                                              int check_finished, double *red) {
+  const bool on = step_wanted(ctrl, check_finished);
+  if (blockIdx.x == 0) {
+    if (threadIdx.x == 0) ctrl[CTRL_ACTIVE] = on ? 1.0 : 0.0;
+    if (on && mode != SETDT_LATER) step_dt<256>(ctrl, parts, nparts, fixed_dt, mode, cfl, red);
+    return;
+  }
+  if (!on) return;
+  const long long total = ghost_shell_cells(p), stride = (long long)(gridDim.x - 1) * 256;
+  for (long long t = (blockIdx.x - 1) * 256LL + threadIdx.x; t < total; t += stride)
+    ghost_shell_element<NV>(U, p, t, copy);
+}
+inline unsigned prologue_blocks(long long ghost_cells) {
+  const long long g = (ghost_cells + 255) / 256;
+  return (unsigned)(1 + (g > 65536 ? 65536 : g));
+}
+// after a step: ++iteration; t += dt (src/shared/SolverBase.cpp:216-218), by one thread of the
+// step's last kernel, whose blocks read only dt and the active flag of the control block.
+// `host` (may be null): the pinned copy that the host reads after a synchronization.
+__device__ __forceinline__ void step_end(double *ctrl, double *host) {
+  const double it = ctrl[CTRL_ITER] + 1.0, t = ctrl[CTRL_T] + ctrl[CTRL_DT];
+  ctrl[CTRL_ITER] = it;
+  ctrl[CTRL_T] = t;
+  if (host) {
+    host[CTRL_ITER] = it;
+    host[CTRL_T] = t;
+    host[CTRL_DT] = ctrl[CTRL_DT];
+    host[CTRL_INVDT] = ctrl[CTRL_INVDT];
+  }
 }
 
 }  // namespace ppk

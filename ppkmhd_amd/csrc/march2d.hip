@@ -21,7 +21,7 @@ namespace march2k {
 template <int RS, int ST, int ISO>
 __global__ void __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(2, 2)))
 k_march2d(const double *__restrict__ Uin, double *__restrict__ Uout, double *__restrict__ parts,
-          DevParams pk, const double *ctrl, int fold) {
+          DevParams pk, double *ctrl, double *host, int fold) {
   if (ctrl[CTRL_ACTIVE] == 0.0) return;
   __shared__ double ring[kWaves * kRing];
   DevParams p = pk;
@@ -31,6 +31,7 @@ k_march2d(const double *__restrict__ Uin, double *__restrict__ Uout, double *__r
   const int w = xcd_remap(blockIdx.x, gridDim.x) * kWaves + wave;
   const Geom g = geom_of(p);
   if (w >= g.waves()) return;  // whole waves only
+  if (w == 0 && threadIdx.x == 0) step_end(ctrl, host);
   const double m = march2d<RS>(Uin, Uout, p, g, w, ctrl[CTRL_DT], fold != 0, ring + wave * kRing);
   if (fold && (threadIdx.x & 63) == 0) parts[w] = m;
 }
@@ -38,13 +39,13 @@ k_march2d(const double *__restrict__ Uin, double *__restrict__ Uout, double *__r
 }  // namespace march2k
 
 hipError_t march2d_godunov(const DevParams &p, const double *Uin, double *Uout, double *parts,
-                           const double *ctrl, int fold_cfl, hipStream_t s, StageTimer *tm) {
+                           double *ctrl, double *host, int fold_cfl, hipStream_t s, StageTimer *tm) {
   using namespace march2k;
   const Geom g = geom_of(p);
   const dim3 grid((unsigned)((g.waves() + kWaves - 1) / kWaves)), block(64 * kWaves);
   if (tm) tm->mark(ST_FUSED_MARCH, true);
   auto launch = [&](auto kernel) {
-    hipLaunchKernelGGL(kernel, grid, block, 0, s, Uin, Uout, parts, p, ctrl, fold_cfl);
+    hipLaunchKernelGGL(kernel, grid, block, 0, s, Uin, Uout, parts, p, ctrl, host, fold_cfl);
   };
   const int minmod = p.slope_type == 1.0 ? 1 : 0, iso = p.cIso > 0 ? 1 : 0;
   auto pick = [&](auto rs) {

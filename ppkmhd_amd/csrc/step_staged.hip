@@ -397,20 +397,11 @@ __global__ void __launch_bounds__(kBlock) k_update(const double *__restrict__ Ui
 }
 
 // ---- time-loop control (single thread) ------------------------------------------------------
-// before a step: stop when SolverBase::finished() holds (src/shared/SolverBase.cpp:195-201)
-// if the step was asked to check
+// before a step: stop when SolverBase::finished() holds, if the step was asked to check
 __global__ void k_begin(double *ctrl, int check_finished) {
-  if (threadIdx.x != 0) return;
-  if (check_finished) {
-    double t = ctrl[CTRL_T], tEnd = ctrl[CTRL_TEND];
-    bool done = t >= (tEnd - 1e-14) || ctrl[CTRL_ITER] >= ctrl[CTRL_NSTEPMAX];
-    ctrl[CTRL_ACTIVE] = done ? 0.0 : 1.0;
-  } else {
-    ctrl[CTRL_ACTIVE] = 1.0;
-  }
+  if (threadIdx.x == 0) ctrl[CTRL_ACTIVE] = step_wanted(ctrl, check_finished) ? 1.0 : 0.0;
 }
-// dt from the CFL partial maxima or the fixed value, clamped to tEnd - t,
-// src/muscl/SolverMHDMuscl.h:737 and src/shared/SolverBase.cpp:173-177.  One block.
+// dt of the step (step_dt).  One block.
 constexpr int kSetDtBlock = 1024;
 __global__ void __launch_bounds__(kSetDtBlock) k_set_dt(double *ctrl,
                                                         const double *__restrict__ parts,
@@ -418,40 +409,19 @@ __global__ void __launch_bounds__(kSetDtBlock) k_set_dt(double *ctrl,
                                                         double cfl) {
   __shared__ double red[kSetDtBlock / 64];
   if (ctrl[CTRL_ACTIVE] == 0.0) return;
-  if (mode == SETDT_FIXED) {
-    // a fixed dt is clamped to tEnd like the CFL one (SolverBase.cpp:173-177), so a run of
-    // fixed steps stops exactly at tEnd
-    if (threadIdx.x == 0) {
-      double dt = fixed_dt;
-      if (ctrl[CTRL_T] + dt > ctrl[CTRL_TEND]) dt = ctrl[CTRL_TEND] - ctrl[CTRL_T];
-      ctrl[CTRL_DT] = dt;
-    }
-    return;
-  }
-  // eight independent loads in flight per thread: the partials can number ~10^5
-  double m[8] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
-  int b = threadIdx.x;
-  for (; b + 7 * kSetDtBlock < nparts; b += 8 * kSetDtBlock) {
-#pragma unroll
-    for (int u = 0; u < 8; ++u) m[u] = fmax(m[u], parts[b + u * kSetDtBlock]);
-  }
-  for (; b < nparts; b += kSetDtBlock) m[0] = fmax(m[0], parts[b]);
-#pragma unroll
-  for (int u = 1; u < 8; ++u) m[0] = fmax(m[0], m[u]);
-  const double mx = block_max(m[0], red);
-  if (threadIdx.x != 0) return;
-  ctrl[CTRL_INVDT] = mx;
-  if (mode == SETDT_CFL) {
-    double dt = cfl / mx;
-    if (ctrl[CTRL_T] + dt > ctrl[CTRL_TEND]) dt = ctrl[CTRL_TEND] - ctrl[CTRL_T];
-    ctrl[CTRL_DT] = dt;
-  }
+  step_dt<kSetDtBlock>(ctrl, parts, nparts, fixed_dt, mode, cfl, red);
 }
-// after a step: ++iteration; t += dt (src/shared/SolverBase.cpp:216-218)
+__global__ void __launch_bounds__(kBlock) k_prologue(double *__restrict__ U,
+                                                     double *__restrict__ copy, DevParams p,
+                                                     double *ctrl,
+                                                     const double *__restrict__ parts, int nparts,
+                                                     double fixed_dt, int mode, double cfl,
+                                                     int check_finished) {
+  __shared__ double red[kBlock / 64];
+  step_prologue<8>(U, copy, p, ctrl, parts, nparts, fixed_dt, mode, cfl, check_finished, red);
+}
 __global__ void k_end(double *ctrl) {
-  if (threadIdx.x != 0 || ctrl[CTRL_ACTIVE] == 0.0) return;
-  ctrl[CTRL_ITER] += 1.0;
-  ctrl[CTRL_T] += ctrl[CTRL_DT];
+  if (threadIdx.x == 0 && ctrl[CTRL_ACTIVE] != 0.0) step_end(ctrl, nullptr);
 }
 
 int grid_for(long long n) {
@@ -472,6 +442,17 @@ hipError_t staged_boundaries(const DevParams &p, double *U, double *copy, const 
   hipLaunchKernelGGL(k_boundaries, dim3(grid_for(ghost_shell_cells(p))), dim3(kBlock), 0, s, U,
                      copy, p, ctrl);
   if (tm) tm->mark(ST_BOUNDARIES, false);
+  return hipGetLastError();
+}
+
+hipError_t staged_prologue(const DevParams &p, double *U, double *copy, double *ctrl,
+                           const double *parts, int nparts, double fixed_dt, int mode, double cfl,
+                           int check_finished, hipStream_t s, StageTimer *tm) {
+  static_assert(kBlock == 256, "step_prologue is written for 256 threads");
+  PPK_TIMED(tm, ST_BOUNDARIES,
+            hipLaunchKernelGGL(k_prologue, dim3(prologue_blocks(ghost_shell_cells(p))),
+                               dim3(kBlock), 0, s, U, copy, p, ctrl, parts, nparts, fixed_dt, mode,
+                               cfl, check_finished));
   return hipGetLastError();
 }
 
