@@ -38,10 +38,8 @@ struct ppk_mlp {
   float *P = nullptr, *m = nullptr, *v = nullptr;
   ppk::MlpPacked *packed = nullptr;
   long long adam_step = 0;
-  // training scratch, sized for the last minibatch
-  uint16_t *scratch = nullptr;
-  float *partials = nullptr;
-  long long scratch_batch = 0;
+  float *partials = nullptr;  // gradient partials of a training step, one per block
+  int partial_blocks = 0;     // blocks it holds
   hipStream_t stream = nullptr;
   std::string err;
 };

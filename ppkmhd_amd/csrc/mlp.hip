@@ -1,13 +1,13 @@
 // Training and evaluation kernels of the surrogate network (layout: mlp.hpp).
 //
-// One training step over a minibatch of B samples (B a multiple of 256):
-//   k_fb      one wavefront per 64 samples: standardise, forward (MFMA), loss gradient,
-//             backward to the pre-activation gradients (MFMA with the transposed weights);
-//             stores the bf16 activations and gradients feature-major for the next kernel
-//   k_wgrad   one block per 256 samples: weight gradients dW = dZ^T H over its samples
-//             (MFMA, the samples are the k dimension) and bias sums, as FP32 partials
-//   k_adam    sums the partials and applies Adam to the FP32 master parameters
-//   k_pack    bf16 MFMA operand copies of the new weights
+// One training step over a minibatch of B samples (B a multiple of 256), two launches:
+//   k_train   one wavefront per 16 samples, 8 wavefronts per block: standardise, forward
+//             (MFMA), loss gradient, backward to the pre-activation gradients (MFMA with the
+//             transposed weights); the bf16 activations and gradients of the block's 128 samples
+//             stay in LDS, feature-major, and the block sums its weight gradients dW = dZ^T H
+//             from there (MFMA, the samples are the k dimension); FP32 partials per block
+//   k_adam    sums the partials, applies Adam to the FP32 master parameters and refreshes the
+//             bf16 operand copies of each weight
 // The loss is the mean over samples and the 8 outputs of (y - (t - mu_out) / sig_out)^2.
 #include <hip/hip_runtime.h>
 
@@ -19,8 +19,12 @@ namespace mlpk {
 
 using namespace mlpd;
 
-constexpr int kWaveSamples = 64;
-constexpr int kChunk = 256;  // samples per k_wgrad block
+constexpr int kWaveSamples = 64;  // inference: samples per wavefront
+constexpr int kTrainWaves = 8, kGroup = 16 * kTrainWaves;  // k_train: samples per pass of a block
+constexpr int kMaxTrainBlocks = 256;  // one per CU; more groups are walked with this stride
+// row stride of the feature-major LDS arrays: 8 samples more than a group, so that the 16 rows
+// of an operand load start 4 banks apart
+constexpr int kSP = kGroup + 8;
 
 // sample index of minibatch slot i of training step `step` (uniform with replacement)
 __device__ __forceinline__ long long pick(unsigned long long seed, long long step, long long i,
@@ -46,39 +50,75 @@ __device__ __forceinline__ void stage_samples(const MlpView &w, const float *X, 
   }
 }
 
-// scratch of one minibatch, feature-major bf16: X 16 x B, H1 128 x B, H2 128 x B, dZ1 128 x B,
-// dZ2 128 x B, dY 8 x B
-struct FbScratch {
-  uint16_t *X, *H1, *H2, *dZ1, *dZ2, *dY;
+struct TrainLds {
+  uint16_t H1[128 * kSP], H2[128 * kSP], Z1[128 * kSP], Z2[128 * kSP];  // activations, gradients
+  uint16_t XT[16 * kSP], DY[16 * kSP];  // features, output gradients (rows 8..15 zero)
+  uint16_t X[kTrainWaves][16 * 16];     // features, sample-major
+  float T[kTrainWaves][16 * 8];         // standardised targets
 };
-__host__ __device__ __forceinline__ FbScratch fb_scratch(uint16_t *base, long long B) {
-  return {base, base + 16 * B, base + 144 * B, base + 272 * B, base + 400 * B, base + 528 * B};
+static_assert(sizeof(TrainLds) <= 160 * 1024, "training block exceeds the LDS of a CU");
+
+__device__ __forceinline__ uint16_t bits_of(__bf16 x) { return __builtin_bit_cast(uint16_t, x); }
+// operand of a 16x16x32 step over samples: lane l holds 8 samples from 8 (l / 16) of row l % 16
+__device__ __forceinline__ v8bf ld_rows(const uint16_t *A, int row, int k) {
+  const int lane = lane_id();
+  return *reinterpret_cast<const v8bf *>(A + (row + (lane & 15)) * kSP + k + 8 * (lane >> 4));
+}
+__device__ __forceinline__ float row_sum(const uint16_t *A, int row, float acc) {
+#pragma unroll 4
+  for (int k = 0; k < kGroup; k += 8) {
+    const v8bf v = *reinterpret_cast<const v8bf *>(A + row * kSP + k);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) acc += (float)v[e];
+  }
+  return acc;
 }
 
-__global__ void __launch_bounds__(256) k_fb(const MlpPacked *__restrict__ net,
-                                            const float *__restrict__ X,
-                                            const float *__restrict__ T, const long long *idx,
-                                            long long n, unsigned long long seed, long long step,
-                                            long long B, uint16_t *scratch, float inv_count) {
-  __shared__ __attribute__((aligned(16))) uint16_t sXall[4][64 * 16];
-  __shared__ float sTall[4][64 * 8];
+// A minibatch of 4096 is 32 blocks of 8 wavefronts.  The time is one group's chain of loads and
+// MFMAs, not work (0.5 GFLOP a step), so a wavefront takes 16 samples only: with 64 per
+// wavefront and the activations in memory between two kernels, 16 blocks each, a step took 117
+// us, now 31 (k_train 27, k_adam 4).
+__global__ void __launch_bounds__(64 * kTrainWaves)
+k_train(const MlpPacked *__restrict__ net, const float *__restrict__ X,
+        const float *__restrict__ T, const long long *idx, long long n, unsigned long long seed,
+        long long step, long long B, float *partials, float inv_count) {
+  __shared__ __attribute__((aligned(16))) TrainLds S;
   const MlpView w = view_of(net);
   const int wave = threadIdx.x >> 6, lane = lane_id(), g = lane >> 4, col = lane & 15;
-  const long long s0 = ((long long)blockIdx.x * 4 + wave) * kWaveSamples;
-  if (s0 >= B) return;
-  uint16_t *sX = sXall[wave];
-  float *sT = sTall[wave];
-  const long long me = s0 + lane;
-  const long long sample = idx ? idx[me] : pick(seed, step, me, n);
-  stage_samples(w, X, T, sample, sX, sT);
-  wave_lds_sync();
-  FbScratch S = fb_scratch(scratch, B);
+  uint16_t *sX = S.X[wave];
+  float *sT = S.T[wave];
+  const int sc = 16 * wave + col;  // this lane's sample column in the feature-major arrays
+  for (int k = threadIdx.x; k < 8 * kSP; k += 64 * kTrainWaves) S.DY[8 * kSP + k] = 0;
+  // weight gradients of this wavefront: dW2 tiles (a, wave), then dW1 tile wave, dW3 tile wave
+  v4f acc[10];
 #pragma unroll
-  for (int i = 0; i < 16; ++i) S.X[(long long)i * B + me] = sX[lane * 16 + i];
+  for (int a = 0; a < 10; ++a) acc[a] = v4f{0.f, 0.f, 0.f, 0.f};
+  float bias = 0.f;  // threads 0..127 b1, 128..255 b2, 256..263 b3
+
 #pragma unroll 1
-  for (int f = 0; f < 4; ++f) {
-    const long long sc = s0 + 16 * f + col;  // the sample of this lane's column
-    const v4s xb = *reinterpret_cast<const v4s *>(sX + (16 * f + col) * 16 + 4 * g);
+  for (long long grp = blockIdx.x; grp < B / kGroup; grp += gridDim.x) {
+    {  // four lanes per sample: four features and two targets each
+      const int s = lane >> 2, part = lane & 3;
+      const long long slot = grp * kGroup + 16 * wave + s;
+      const long long sample = idx ? idx[slot] : pick(seed, step, slot, n);
+      const float4 x = *reinterpret_cast<const float4 *>(X + sample * kMlpIn + 4 * part);
+      const float2 t = *reinterpret_cast<const float2 *>(T + sample * kMlpOut + 2 * part);
+      const float xv[4] = {x.x, x.y, x.z, x.w}, tv[2] = {t.x, t.y};
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int i = 4 * part + e;
+        const uint16_t v = bf16_bits((xv[e] - w.mu_in[i]) * w.isig_in[i]);
+        sX[s * 16 + i] = v;
+        S.XT[i * kSP + 16 * wave + s] = v;
+      }
+#pragma unroll
+      for (int e = 0; e < 2; ++e) {
+        const int o = 2 * part + e;
+        sT[s * 8 + o] = (tv[e] - w.mu_out[o]) / w.sig_out[o];
+      }
+    }
+    wave_lds_sync();
+    const v4s xb = *reinterpret_cast<const v4s *>(sX + col * 16 + 4 * g);
     v8bf h1b[4], h2b[4];
     unsigned m1, m2;
     v4f y;
@@ -91,21 +131,17 @@ __global__ void __launch_bounds__(256) k_fb(const MlpPacked *__restrict__ net,
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
         const int h = mlp_feat(q, g, e);
-        __bf16 a = h1b[q][e], b = h2b[q][e];
-        uint16_t ua, ub;
-        __builtin_memcpy(&ua, &a, 2);
-        __builtin_memcpy(&ub, &b, 2);
-        S.H1[(long long)h * B + sc] = ua;
-        S.H2[(long long)h * B + sc] = ub;
+        S.H1[h * kSP + sc] = bits_of(h1b[q][e]);
+        S.H2[h * kSP + sc] = bits_of(h2b[q][e]);
       }
     // loss gradient (outputs 4g + j of sample col)
     v4s dyb;
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       const int o = 4 * g + j;
-      const float dy = o < 8 ? 2.f * (y[j] - sT[(16 * f + col) * 8 + o]) * inv_count : 0.f;
+      const float dy = o < 8 ? 2.f * (y[j] - sT[col * 8 + o]) * inv_count : 0.f;
       dyb[j] = bf16s(dy);
-      if (o < 8) S.dY[(long long)o * B + sc] = (uint16_t)dyb[j];
+      if (o < 8) S.DY[o * kSP + sc] = (uint16_t)dyb[j];
     }
     // dH2 = W3^T dY, dZ2 = dH2 * (z2 > 0), packed in pairs as the B operands of dH1
     v8bf db[4];
@@ -120,7 +156,7 @@ __global__ void __launch_bounds__(256) k_fb(const MlpPacked *__restrict__ net,
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
           t[h][j] = (m2 >> (4 * r + j)) & 1u ? c[j] : 0.f;
-          S.dZ2[(long long)(16 * r + 4 * g + j) * B + sc] = bf16_bits(t[h][j]);
+          S.Z2[(16 * r + 4 * g + j) * kSP + sc] = bf16_bits(t[h][j]);
         }
       }
       db[q] = pack_pair(t[0], t[1]);
@@ -133,79 +169,81 @@ __global__ void __launch_bounds__(256) k_fb(const MlpPacked *__restrict__ net,
       for (int q = 0; q < 4; ++q) c = mfma_k32(ld_a32(wf.A2T, r * 4 + q, lane), db[q], c);
 #pragma unroll
       for (int j = 0; j < 4; ++j)
-        S.dZ1[(long long)(16 * r + 4 * g + j) * B + sc] =
+        S.Z1[(16 * r + 4 * g + j) * kSP + sc] =
             bf16_bits((m1 >> (4 * r + j)) & 1u ? c[j] : 0.f);
     }
-  }
-}
-
-// one 16x16 tile of sum_s A[rowA + i][s] * Bm[rowB + n][s] over samples [s0, s0 + kChunk)
-__device__ __forceinline__ v4f tile_gemm(const uint16_t *A, int rowA, int nrowA,
-                                         const uint16_t *Bm, int rowB, long long B, long long s0) {
-  const int lane = lane_id(), g = lane >> 4, col = lane & 15;
-  v4f c = {0.f, 0.f, 0.f, 0.f};
-  const int ra = rowA + col;
-#pragma unroll 2
-  for (int k = 0; k < kChunk; k += 32) {
-    v8bf a, b;
-    const long long off = s0 + k + 8 * g;
-    if (ra < nrowA)
-      a = *reinterpret_cast<const v8bf *>(A + (long long)ra * B + off);
-    else
-      a = v8bf{};
-    b = *reinterpret_cast<const v8bf *>(Bm + (long long)(rowB + col) * B + off);
-    c = mfma_k32(a, b, c);
-  }
-  return c;
-}
-
-__global__ void __launch_bounds__(256) k_wgrad(const uint16_t *scratch, long long B,
-                                               float *partials) {
-  const FbScratch S = fb_scratch(const_cast<uint16_t *>(scratch), B);
-  const long long s0 = (long long)blockIdx.x * kChunk;
-  float *P = partials + (long long)blockIdx.x * kMlpTrained;
-  const int wave = threadIdx.x >> 6, lane = lane_id(), g = lane >> 4, col = lane & 15;
-  // 80 tiles: dW2 64 (a, b), dW1 8 (a), dW3 8 (b); 20 per wave
-  for (int t = wave; t < 80; t += 4) {
-    if (t < 64) {
-      const int a = t / 8, b = t % 8;
-      const v4f c = tile_gemm(S.dZ2, 16 * a, 128, S.H1, 16 * b, B, s0);
+    __syncthreads();
+    // gradients over the group's samples
 #pragma unroll
-      for (int j = 0; j < 4; ++j) P[kMlpW2 + (16 * a + 4 * g + j) * 128 + 16 * b + col] = c[j];
-    } else if (t < 72) {
-      const int a = t - 64;
-      const v4f c = tile_gemm(S.dZ1, 16 * a, 128, S.X, 0, B, s0);
+    for (int k = 0; k < kGroup; k += 32) {
+      const v8bf h1 = ld_rows(S.H1, 16 * wave, k);
 #pragma unroll
-      for (int j = 0; j < 4; ++j) P[kMlpW1 + (16 * a + 4 * g + j) * 16 + col] = c[j];
-    } else {
-      const int b = t - 72;
-      const v4f c = tile_gemm(S.dY, 0, 8, S.H2, 16 * b, B, s0);
-#pragma unroll
-      for (int j = 0; j < 4; ++j)
-        if (4 * g + j < 8) P[kMlpW3 + (4 * g + j) * 128 + 16 * b + col] = c[j];
+      for (int a = 0; a < 8; ++a) acc[a] = mfma_k32(ld_rows(S.Z2, 16 * a, k), h1, acc[a]);
+      acc[8] = mfma_k32(ld_rows(S.Z1, 16 * wave, k), ld_rows(S.XT, 0, k), acc[8]);
+      acc[9] = mfma_k32(ld_rows(S.DY, 0, k), ld_rows(S.H2, 16 * wave, k), acc[9]);
     }
+    const int f = threadIdx.x;
+    if (f < 256)
+      bias = row_sum(f < 128 ? S.Z1 : S.Z2, f & 127, bias);
+    else if (f < 264)
+      bias = row_sum(S.DY, f - 256, bias);
+    __syncthreads();
   }
-  // bias gradients: sums of the stored bf16 gradients over the chunk
+
+  float *P = partials + (long long)blockIdx.x * kMlpTrained;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const int i = 4 * g + j;
+#pragma unroll
+    for (int a = 0; a < 8; ++a) P[kMlpW2 + (16 * a + i) * 128 + 16 * wave + col] = acc[a][j];
+    P[kMlpW1 + (16 * wave + i) * 16 + col] = acc[8][j];
+    if (i < 8) P[kMlpW3 + i * 128 + 16 * wave + col] = acc[9][j];
+  }
   const int f = threadIdx.x;
-  {
-    const uint16_t *src = f < 128 ? S.dZ1 + (long long)f * B : S.dZ2 + (long long)(f - 128) * B;
-    float acc = 0.f;
-    for (int s = 0; s < kChunk; ++s) acc += bf16_value(src[s0 + s]);
-    P[(f < 128 ? kMlpB1 + f : kMlpB2 + f - 128)] = acc;
-  }
-  if (f < 8) {
-    float acc = 0.f;
-    for (int s = 0; s < kChunk; ++s) acc += bf16_value(S.dY[(long long)f * B + s0 + s]);
-    P[kMlpB3 + f] = acc;
+  if (f < 264) P[f < 128 ? kMlpB1 + f : (f < 256 ? kMlpB2 + f - 128 : kMlpB3 + f - 256)] = bias;
+}
+
+// the packed copies of trained parameter i (the inverse of pack_weight)
+__device__ __forceinline__ void repack(MlpPacked *net, int i, float p) {
+  const uint16_t v = bf16_bits(p);
+  auto feat = [](int f, int &q, int &g, int &e) {  // inverse of mlp_feat
+    q = f >> 5;
+    const int r = f & 31;
+    g = (r & 15) >> 2;
+    e = (r & 3) + (r < 16 ? 0 : 4);
+  };
+  int q, g, e;
+  if (i < kMlpB1) {
+    const int o = i >> 4, c = i & 15;
+    net->A1[o >> 4][(c >> 2) * 16 + (o & 15)][c & 3] = v;
+  } else if (i < kMlpW2) {
+    net->b1[i - kMlpB1] = p;
+  } else if (i < kMlpB2) {
+    const int o = (i - kMlpW2) >> 7, f = (i - kMlpW2) & 127;
+    feat(f, q, g, e);
+    net->A2[o >> 4][q][g * 16 + (o & 15)][e] = v;
+    feat(o, q, g, e);
+    net->A2T[f >> 4][q][g * 16 + (f & 15)][e] = v;
+  } else if (i < kMlpW3) {
+    net->b2[i - kMlpB2] = p;
+  } else if (i < kMlpB3) {
+    const int o = (i - kMlpW3) >> 7, f = (i - kMlpW3) & 127;
+    feat(f, q, g, e);
+    net->A3[q][g * 16 + o][e] = v;
+    net->A3T[f >> 4][(o >> 2) * 16 + (f & 15)][o & 3] = v;
+  } else {
+    net->b3[i - kMlpB3] = p;
   }
 }
 
-__global__ void k_adam(const float *partials, int nchunks, float *P, float *m, float *v,
-                       float *grad_out, int step, float lr, float beta1, float beta2, float eps) {
+__global__ void __launch_bounds__(64)
+k_adam(const float *__restrict__ partials, int nparts, float *P, float *m, float *v,
+       float *grad_out, MlpPacked *net, int step, float lr, float beta1, float beta2, float eps) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= kMlpTrained) return;
   float gsum = 0.f;
-  for (int c = 0; c < nchunks; ++c) gsum += partials[(long long)c * kMlpTrained + i];
+#pragma unroll 16
+  for (int c = 0; c < nparts; ++c) gsum += partials[(long long)c * kMlpTrained + i];
   if (grad_out) grad_out[i] = gsum;
   if (lr == 0.f) return;  // gradient only
   const float mi = beta1 * m[i] + (1.f - beta1) * gsum;
@@ -214,7 +252,9 @@ __global__ void k_adam(const float *partials, int nchunks, float *P, float *m, f
   v[i] = vi;
   const float mh = mi / (1.f - __powf(beta1, (float)step));
   const float vh = vi / (1.f - __powf(beta2, (float)step));
-  P[i] -= lr * mh / (sqrtf(vh) + eps);
+  const float p = P[i] - lr * mh / (sqrtf(vh) + eps);
+  P[i] = p;
+  repack(net, i, p);
 }
 
 __global__ void k_pack(const float *P, MlpPacked *net) {
@@ -309,24 +349,23 @@ __global__ void __launch_bounds__(256) k_moments(const float *__restrict__ X,
 // ---- launchers (mlp_kernels.hpp) -----------------------------------------------------------
 namespace mlp {
 
-size_t fb_scratch_elems(long long B) { return (size_t)536 * B; }
+int train_blocks(long long B) {
+  const long long g = B / mlpk::kGroup;
+  return (int)(g < mlpk::kMaxTrainBlocks ? g : mlpk::kMaxTrainBlocks);
+}
 
-hipError_t train_step(const MlpPacked *net, float *P, float *m, float *v, const float *X,
+hipError_t train_step(MlpPacked *net, float *P, float *m, float *v, const float *X,
                       const float *T, const long long *idx, long long n, unsigned long long seed,
-                      long long step, long long B, uint16_t *scratch, float *partials,
-                      float *grad_out, float lr, hipStream_t s) {
+                      long long step, long long B, float *partials, float *grad_out, float lr,
+                      hipStream_t s) {
   using namespace mlpk;
-  if (B % kChunk) return hipErrorInvalidValue;
+  if (B < kGroup || B % kGroup) return hipErrorInvalidValue;
   const float inv_count = 1.f / (float)(B * kMlpOut);
-  hipLaunchKernelGGL(k_fb, dim3((unsigned)(B / 256)), dim3(256), 0, s, net, X, T, idx, n, seed,
-                     step, B, scratch, inv_count);
-  hipLaunchKernelGGL(k_wgrad, dim3((unsigned)(B / kChunk)), dim3(256), 0, s, scratch, B, partials);
-  hipLaunchKernelGGL(k_adam, dim3((kMlpTrained + 255) / 256), dim3(256), 0, s, partials,
-                     (int)(B / kChunk), P, m, v, grad_out, (int)(step + 1), lr, 0.9f, 0.999f,
-                     1e-8f);
-  if (lr != 0.f)
-    hipLaunchKernelGGL(k_pack, dim3((kPackWeights + 255) / 256), dim3(256), 0, s, P,
-                       const_cast<MlpPacked *>(net));
+  const int nb = train_blocks(B);
+  hipLaunchKernelGGL(k_train, dim3((unsigned)nb), dim3(64 * kTrainWaves), 0, s, net, X, T,
+                     idx, n, seed, step, B, partials, inv_count);
+  hipLaunchKernelGGL(k_adam, dim3((kMlpTrained + 63) / 64), dim3(64), 0, s, partials, nb, P, m, v,
+                     grad_out, net, (int)(step + 1), lr, 0.9f, 0.999f, 1e-8f);
   return hipGetLastError();
 }
 

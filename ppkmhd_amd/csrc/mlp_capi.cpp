@@ -45,7 +45,7 @@ double uniform(unsigned long long &s) { return (splitmix(s) >> 11) * (1.0 / 9007
 
 void free_net(ppk_mlp_t *n) {
   for (void *p : {(void *)n->P, (void *)n->m, (void *)n->v, (void *)n->packed,
-                  (void *)n->scratch, (void *)n->partials})
+                  (void *)n->partials})
     if (p) (void)hipFree(p);
   if (n->stream) (void)hipStreamDestroy(n->stream);
 }
@@ -66,16 +66,15 @@ int upload_params(ppk_mlp_t *n, const float *P) {
   return PPK_OK;
 }
 
+// gradient partials of a training step on B samples (bounded: one block per CU at most)
 int ensure_scratch(ppk_mlp_t *n, long long B) {
-  if (n->scratch_batch >= B) return PPK_OK;
-  if (n->scratch) (void)hipFree(n->scratch);
+  const int blocks = ppk::mlp::train_blocks(B);
+  if (n->partial_blocks >= blocks) return PPK_OK;
   if (n->partials) (void)hipFree(n->partials);
-  n->scratch = nullptr;
   n->partials = nullptr;
-  n->scratch_batch = 0;
-  NHIP(n, hipMalloc(&n->scratch, sizeof(uint16_t) * ppk::mlp::fb_scratch_elems(B)));
-  NHIP(n, hipMalloc(&n->partials, sizeof(float) * (size_t)(B / 256) * ppk::kMlpTrained));
-  n->scratch_batch = B;
+  n->partial_blocks = 0;
+  NHIP(n, hipMalloc(&n->partials, sizeof(float) * (size_t)blocks * ppk::kMlpTrained));
+  n->partial_blocks = blocks;
   return PPK_OK;
 }
 
@@ -272,7 +271,7 @@ int ppk_mlp_train(ppk_mlp_t *net, const ppk_faceset_t *set, int steps, int batch
   if (rc != PPK_OK) return rc;
   for (int i = 0; i < steps; ++i) {
     NHIP(net, ppk::mlp::train_step(net->packed, net->P, net->m, net->v, set->X, set->T, nullptr,
-                                   (long long)set->n, seed, net->adam_step, batch, net->scratch,
+                                   (long long)set->n, seed, net->adam_step, batch,
                                    net->partials, nullptr, lr, net->stream));
     ++net->adam_step;
   }
@@ -302,7 +301,7 @@ int ppk_mlp_gradient(ppk_mlp_t *net, const float *X, const float *T, size_t n, f
   if (e == hipSuccess) e = hipMemcpy(idx, hidx.data(), sizeof(long long) * n, hipMemcpyHostToDevice);
   if (e == hipSuccess)
     e = ppk::mlp::train_step(net->packed, net->P, net->m, net->v, dX, dT, idx, (long long)n, 0, 0,
-                             (long long)n, net->scratch, net->partials, dG, 0.f, net->stream);
+                             (long long)n, net->partials, dG, 0.f, net->stream);
   if (e == hipSuccess) e = hipStreamSynchronize(net->stream);
   if (e == hipSuccess) e = hipMemcpy(grad, dG, sizeof(float) * count, hipMemcpyDeviceToHost);
   for (void *p : {(void *)dX, (void *)dT, (void *)dG, (void *)idx})

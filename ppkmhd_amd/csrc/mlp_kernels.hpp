@@ -12,16 +12,16 @@
 namespace ppk {
 namespace mlp {
 
-// bf16 elements of the per-minibatch scratch of train_step
-size_t fb_scratch_elems(long long B);
+// blocks (gradient partials) of a training step on B samples: at most one per CU
+int train_blocks(long long B);
 // One Adam step on a minibatch of B samples (B % 256 == 0) drawn from the n samples X, T
 // (idx: explicit sample indices, or null to draw them from `seed` and `step`).  partials:
-// (B / 256) x 19720 floats.  grad_out (optional): the summed gradient.  lr == 0 computes the
-// gradient only and leaves the parameters unchanged.
-hipError_t train_step(const MlpPacked *net, float *P, float *m, float *v, const float *X,
+// train_blocks(B) x 19720 floats.  grad_out (optional): the summed gradient.  lr == 0 computes
+// the gradient only and leaves the parameters unchanged.
+hipError_t train_step(MlpPacked *net, float *P, float *m, float *v, const float *X,
                       const float *T, const long long *idx, long long n, unsigned long long seed,
-                      long long step, long long B, uint16_t *scratch, float *partials,
-                      float *grad_out, float lr, hipStream_t s);
+                      long long step, long long B, float *partials, float *grad_out, float lr,
+                      hipStream_t s);
 hipError_t pack(const float *P, MlpPacked *net, hipStream_t s);
 int infer_blocks(long long n);
 // standardised outputs Y[n][8] (optional) and per-block squared-error sums against T

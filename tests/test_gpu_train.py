@@ -1,0 +1,55 @@
+"""The training kernel at the edges of its grouping (128 samples per block and pass, at most 256
+blocks, larger minibatches walked by stride), against the bf16-rounding oracle and against
+itself: a sample set given twice has the same gradient.  The operand copies that training leaves
+are those of its parameters."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def net_and_samples(n, seed=5):
+    from ppkmhd_amd import surrogate as S
+    rng = np.random.default_rng(seed)
+    X = rng.standard_normal((n, 16)).astype(np.float32)
+    T = np.tanh(X[:, :8] * X[:, 8:]).astype(np.float32)
+    net = S.MLP(seed)
+    return S, net, X, T
+
+
+def rel(a, b):
+    return np.linalg.norm(a - b) / np.linalg.norm(b)
+
+
+@pytest.mark.parametrize("n", [256, 512, 33024])
+def test_gradient_matches_oracle(gpu, n):
+    from oracle import surrogate_oracle as O
+    S, net, X, T = net_and_samples(n)
+    g = net.gradient(X, T)
+    ref = O.mlp_grad(net.get_params(), X, T)
+    # FP32 sums of n bf16 products in any order: sqrt(n) 2^-24 and the roundings of dy, dz that a
+    # last-bit difference before them flips (bar of the gradient test, 1e-3 per block of weights)
+    for lo, hi in ((S.W1, S.B1), (S.B1, S.W2), (S.W2, S.B2), (S.B2, S.W3), (S.W3, S.B3),
+                   (S.B3, S.N_TRAINED)):
+        assert rel(g[lo:hi], ref[lo:hi]) < 1e-3
+
+
+def test_more_groups_than_blocks(gpu):
+    """65536 samples are 512 groups in 256 blocks: twice the same 32768 samples (256 groups), so
+    the mean gradient is the same to FP32 rounding of the sums (2^16 terms: 2^-24 x 2^8)."""
+    S, net, X, T = net_and_samples(32768)
+    one = net.gradient(X, T)
+    two = net.gradient(np.concatenate([X, X]), np.concatenate([T, T]))
+    assert rel(two, one) < 2.0 ** -16
+
+
+def test_packed_copies_follow_training(gpu):
+    S, net, X, T = net_and_samples(3000)
+    fs = S.FaceSet(3000)
+    fs.append(X, T)
+    net.standardize(fs)
+    net.train(fs, 7, batch=768, lr=1e-3, seed=3)
+    fresh = S.MLP(99)
+    fresh.set_params(net.get_params())
+    assert np.array_equal(net.infer(X), fresh.infer(X))
+    assert np.array_equal(net.gradient(X[:512], T[:512]), fresh.gradient(X[:512], T[:512]))
