@@ -428,16 +428,20 @@ __global__ void __launch_bounds__(kWaves2 * 64, MINW) k_hfused2d(const double *_
 }
 
 // ---- fused 3D: a block of 8 waves, 16 rows of 32 columns stacked along y, marches along z --
-// Thread t holds row r = t / 32 (two rows per wave), j = gw + 12 * by + r - 2, and column
-// c = t % 32, i = gw + 28 * bx + c - 2; rows 2..13 and columns 2..29 are the block's output
-// (32-wide rows: 336 output cells per block and plane, against 240 with one 64-wide row per
-// wave).  x neighbours come from LDS and shuffles within the 32 lanes of a row.  At slope
-// plane s each thread keeps Q(s-1), Q(s),
-// Q(s+1) of its column in registers; plane s of Q goes through LDS for the x and y
-// neighbours, the upper y-face states of each row through LDS to the row above, and the y
-// fluxes back through LDS to the row below.  The z face below plane s uses the upper z state
-// of plane s-1 kept in registers, so the update of (i, j, s-1) completes at plane s.
+// Thread t holds row r = t / 32 (two rows per wave), j = gw + 14 * by + r - 1, and column
+// c = t % 32, i = gw + 30 * bx + c - 1; rows 1..14 and columns 1..30 are the block's output.
+// At slope plane s each thread keeps Q(s-1), Q(s), Q(s+1) of its column in registers; plane s
+// of Q goes through LDS for the x and y neighbours, with the ring of cells around the block's
+// columns, which the first 96 threads load and convert besides their own (82 % of the threads
+// carry output; with the ring held by threads of its own, 28 x 12 of 32 x 16, it was 66 %).
+// The upper y-face states of each row go through LDS to the row above, and the y fluxes back
+// to the row below; x states and fluxes pass by shuffles within the 32 lanes of a row.  The z
+// face below plane s uses the upper z state of plane s-1 kept in registers, so the update of
+// (i, j, s-1) completes at plane s.  The states of plane s+2 are loaded a plane ahead.
 constexpr int kW3 = kHydroWaves3;
+constexpr int kRW3 = kHydroRowW3, kNR3 = kHydroBlockRows3;  // columns and rows of threads
+constexpr int kRing3 = 2 * (kRW3 + kNR3);                   // cells around them, corners not used
+static_assert(kRing3 <= kW3 * 64, "one ring cell per thread");
 
 template <int NV, int RS, int MINW, int GR>
 __global__ void __launch_bounds__(kW3 * 64, MINW) k_hfused3d(const double *__restrict__ Uin,
@@ -445,9 +449,10 @@ __global__ void __launch_bounds__(kW3 * 64, MINW) k_hfused3d(const double *__res
                                                        double *__restrict__ parts,
                                                        double *ctrl, double *host,
                                                        int fold_cfl) {
-  constexpr int RW = kHydroRowW3, NR = kHydroBlockRows3;
-  __shared__ double sQ[2][NV][NR][RW];  // Q of plane s (parity s & 1), later the y fluxes
-  __shared__ double sT[NV][NR][RW];     // upper y-face states of plane s
+  constexpr int RW = kRW3, NR = kNR3;
+  // Q of plane s (parity s & 1) with its ring, origin (-1, -1), later the y fluxes
+  __shared__ double sQ[2][NV][NR + 2][RW + 2];
+  __shared__ double sT[NV][NR][RW];  // upper y-face states of plane s
   __shared__ double red[kW3];
   if (!active(ctrl)) return;
   if (blockIdx.x == 0 && threadIdx.x == 0) step_end(ctrl, host);
@@ -459,29 +464,37 @@ __global__ void __launch_bounds__(kW3 * 64, MINW) k_hfused3d(const double *__res
   const int bx = blockIdx.x % nsx;
   const int by = (blockIdx.x / nsx) % nsy;
   const int bz = blockIdx.x / (nsx * nsy);
-  const int i = h.gw + bx * kHydroCols3 + lane - 2;
-  const int j = h.gw + by * kHydroRows3 + ly - 2;
-  const int ic = i < h.isize ? i : h.isize - 1;  // clamped halo, never output
-  const int jc = j < h.jsize ? j : h.jsize - 1;
+  const int i0 = h.gw + bx * kHydroCols3 - 1, j0 = h.gw + by * kHydroRows3 - 1;
+  const int i = i0 + lane, j = j0 + ly;
+  // cells past the box: clamped, no output depends on them
+  auto column = [&](int ii, int jj) {
+    return (long long)(jj < h.jsize ? jj : h.jsize - 1) * h.isize +
+           (ii < h.isize ? ii : h.isize - 1);
+  };
   const int k0 = h.gw + bz * KH;
   const int k1 = min(k0 + KH, h.gw + h.nz);
-  const bool slope_row = ly >= 1 && ly <= NR - 2;
-  const bool yface_row = ly >= 2 && ly <= NR - 2;
-  const bool out_row = ly >= 2 && ly < 2 + kHydroRows3;
-  const bool out = out_row && lane >= 2 && lane < 2 + kHydroCols3 && i < h.gw + h.nx &&
+  const bool out_row = ly >= 1 && ly < 1 + kHydroRows3;
+  const bool out = out_row && lane >= 1 && lane < 1 + kHydroCols3 && i < h.gw + h.nx &&
                    j < h.gw + h.ny;
+  // ring cell of this thread: rows -1 and NR, then columns -1 and RW
+  const int rn = threadIdx.x;
+  const bool ring = rn < kRing3;
+  const int rq = rn - 2 * RW;
+  const int ry = rn < 2 * RW ? (rn < RW ? -1 : NR) : rq % NR;
+  const int rx = rn < 2 * RW ? rn % RW : (rq < NR ? -1 : RW);
   const long long vs = h.vstride;
-  const long long col = (long long)jc * h.isize + ic;
+  const long long col = column(i, j), rcol = ring ? column(i0 + rx, j0 + ry) : col;
   const double dt = ctrl[CTRL_DT];
   const double dtdx = dt / h.dx, dtdy = dt / h.dy, dtdz = dt / h.dz, hdt = 0.5 * dt;
   const hyd::HydroPar &P = h.P;
-  const int lm = lane > 0 ? lane - 1 : 0, lp = lane < RW - 1 ? lane + 1 : RW - 1;
 
-  HSt<NV> qm, q0, u0, t;
+  HSt<NV> qm, q0, u0, t, un, ur;
   double c, rho_prev = 0.0;  // density of (i, j, s-1) before the step, for the gravity source
   load(Uin, vs, (long long)(k0 - 2) * h.plane + col, t);
   hyd::prims(t, P, c, qm);
   load(Uin, vs, (long long)(k0 - 1) * h.plane + col, u0);
+  load(Uin, vs, (long long)k0 * h.plane + col, un);
+  if (ring) load(Uin, vs, (long long)(k0 - 1) * h.plane + rcol, ur);
   hyd::prims(u0, P, c, q0);
   // gravity field of the plane the face states are built for, and of the plane being finished
   G3 g0 = cell_g<GR, NV>(h, (long long)(k0 - 1) * h.plane + col), g_prev = g0;
@@ -490,22 +503,30 @@ __global__ void __launch_bounds__(kW3 * 64, MINW) k_hfused3d(const double *__res
 #pragma unroll 1
   for (int s = k0 - 1; s <= k1; ++s) {
     const int b = s & 1;
-    HSt<NV> un, qp;
-    load(Uin, vs, (long long)(s + 1) * h.plane + col, un);
-    hyd::prims(un, P, c, qp);
-    const G3 gn = cell_g<GR, NV>(h, (long long)(s + 1) * h.plane + col);
+    HSt<NV> qp;
 #pragma unroll
-    for (int v = 0; v < NV; ++v) sQ[b][v][ly][lane] = q0[v];
+    for (int v = 0; v < NV; ++v) sQ[b][v][ly + 1][lane + 1] = q0[v];
+    if (ring) {
+      HSt<NV> qr;
+      hyd::prims(ur, P, c, qr);
+#pragma unroll
+      for (int v = 0; v < NV; ++v) sQ[b][v][ry + 1][rx + 1] = qr[v];
+      if (s < k1) load(Uin, vs, (long long)(s + 1) * h.plane + rcol, ur);
+    }
+    hyd::prims(un, P, c, qp);
+    const HSt<NV> u1 = un;  // state of plane s+1, the next update's input
+    if (s < k1) load(Uin, vs, (long long)(s + 2) * h.plane + col, un);
+    const G3 gn = cell_g<GR, NV>(h, (long long)(s + 1) * h.plane + col);
     __syncthreads();
     HSt<NV> dX, dY, dZ, s0;
-    if (slope_row) {
+    {
       HSt<NV> qxm, qxp, qym, qyp;
 #pragma unroll
       for (int v = 0; v < NV; ++v) {
-        qxm[v] = sQ[b][v][ly][lm];
-        qxp[v] = sQ[b][v][ly][lp];
-        qym[v] = sQ[b][v][ly - 1][lane];
-        qyp[v] = sQ[b][v][ly + 1][lane];
+        qxm[v] = sQ[b][v][ly + 1][lane];
+        qxp[v] = sQ[b][v][ly + 1][lane + 2];
+        qym[v] = sQ[b][v][ly][lane + 1];
+        qyp[v] = sQ[b][v][ly + 2][lane + 1];
       }
       hyd::slopes(q0, qxp, qxm, qyp, qym, qp, qm, P, dX, dY, dZ);
       hyd::sources(q0, dX, dY, dZ, P.gamma0, s0);
@@ -529,7 +550,7 @@ __global__ void __launch_bounds__(kW3 * 64, MINW) k_hfused3d(const double *__res
 #pragma unroll
       for (int v = 0; v < NV; ++v) fz[v] = fz[v] * dtdz;
     }
-    if (plane_out && yface_row) {  // y face below row j, flux into the Q slot of plane s
+    if (plane_out && ly >= 1) {  // y face below row j, flux into the Q slot of plane s
       HSt<NV> ql, qr, fy;
 #pragma unroll
       for (int v = 0; v < NV; ++v) ql[v] = sT[v][ly - 1][lane];
@@ -540,7 +561,7 @@ __global__ void __launch_bounds__(kW3 * 64, MINW) k_hfused3d(const double *__res
       hyd::riemann_rs<RS>(ql, qr, fy, P);
       swap_normal(fy, 1);
 #pragma unroll
-      for (int v = 0; v < NV; ++v) sQ[b][v][ly][lane] = fy[v] * dtdy;
+      for (int v = 0; v < NV; ++v) sQ[b][v][ly + 1][lane + 1] = fy[v] * dtdy;
     }
     if (plane_out && out_row) {  // x face left of column i
       HSt<NV> xmin, xmax, xl;
@@ -572,8 +593,8 @@ __global__ void __launch_bounds__(kW3 * 64, MINW) k_hfused3d(const double *__res
           double o = u0[v];
           o += fx[v];
           o -= fxr;
-          o += sQ[b][v][ly][lane];
-          o -= sQ[b][v][ly + 1][lane];
+          o += sQ[b][v][ly + 1][lane + 1];
+          o -= sQ[b][v][ly + 2][lane + 1];
           o += fz[v];
           o_prev[v] = o;
         }
@@ -581,13 +602,11 @@ __global__ void __launch_bounds__(kW3 * 64, MINW) k_hfused3d(const double *__res
         g_prev = g0;
       }
     }
-    if (slope_row) {
-      hyd::face_state(q0, dZ, s0, dtdz, true, P.smallr, zmax_prev);
-      gravity_predict<GR>(zmax_prev, g0, h, hdt);
-    }
+    hyd::face_state(q0, dZ, s0, dtdz, true, P.smallr, zmax_prev);
+    gravity_predict<GR>(zmax_prev, g0, h, hdt);
     qm = q0;
     q0 = qp;
-    u0 = un;
+    u0 = u1;
     g0 = gn;
   }
   if (fold_cfl) {

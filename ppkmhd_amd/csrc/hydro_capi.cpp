@@ -131,11 +131,54 @@ HydroDev make_hydro_dev(const ppk_mhd_params &p) {
   d.cfl = p.cfl;
   d.dxmin = p.dim == 3 ? std::fmin(std::fmin(p.dx, p.dy), p.dz) : std::fmin(p.dx, p.dy);
   d.idxmin = 1.0 / d.dxmin;
-  // tuning knob: output rows (2D) / planes (3D) of one marching wave / block
-  const char *strip = std::getenv("PPKMHD_HYDRO_STRIP");
-  const int rows = strip ? std::atoi(strip) : 0;
-  d.strip_rows = rows > 0 ? rows : (p.dim == 3 ? 48 : 64);  // measured best at 8192 x 4096 / 512 x 384 x 256
+  d.strip_rows = 1;  // the handle picks it (hydro_strip_rows)
   return d;
+}
+
+// Output rows (2D) / planes (3D) of one marching wave / block: few give many waves or blocks to
+// fill the GPU with, but each starts with about two rows or planes that it does not output.
+// The estimates are in us per row or plane; measured per step (MI355X, HLLC, best in brackets):
+//   2D  64^2     64 rows 114, 8 rows 23, [1 row 12]
+//       1024^2   64 rows 116, [6 rows 44], 12 rows 46, 1 row 69
+//       4096x2048  128 rows 365, 64 rows 270, [20 rows 225], 47 rows 227
+//   3D  64^3     48 planes 252, 8 planes 58, [4 planes 41], 1 plane 63
+//       256x192x128  48 planes 454, [64 planes 381], 16 planes 400, 1 plane 866
+// (48 planes and 64 rows were the fixed values.)
+int hydro_strip_rows(const HydroDev &d, int cus) {
+  if (cus <= 0) cus = 256;
+  const int n = d.dim == 3 ? d.nz : d.ny;
+  const auto up = [](double a, double b) { return std::ceil(a / b); };
+  int pick = 1;
+  double best = 0.0;
+  for (int r = 1; r <= n; ++r) {
+    double t;
+    if (d.dim == 2) {
+      // one wave per SIMD takes 1.6 us a row, more share its issue slots (1.35 to 1.4 each)
+      const double x = up(d.nx, kHydroCols) * up(d.ny, r) / (4.0 * cus);
+      t = (r + 2.7) * 1.62;
+      if (x > 1.0) t = std::fmax(t, (r + 1.6) * (x > 3.0 ? 1.35 * (x + 0.5) : 1.4 * std::ceil(x)));
+    } else {
+      // one block per CU at a time: whole rounds of the full-length blocks, the last strips'
+      // shorter blocks beside or after the last round
+      const double cols = up(d.nx, kHydroCols3) * up(d.ny, kHydroRows3);
+      const int rem = d.nz % r;
+      const double full = cols * (d.nz / r), part = rem ? cols : 0.0;
+      const double F = r + 2.4, S = rem + 2.4;
+      const double left = full - std::floor(full / cus) * cus;
+      t = std::floor(full / cus) * F;
+      double rest = part;
+      if (left > 0.0) {
+        t += F;
+        rest = std::fmax(0.0, part - std::floor(F / S) * (cus - left));
+      }
+      t += up(rest, cus) * S;
+    }
+    if (best == 0.0 || t < best) {
+      best = t;
+      pick = r;
+    }
+  }
+  return pick;
 }
 
 // The 19 four-quadrant 2D Riemann configurations of Lax & Liu (SIAM J. Sci. Comput. 19(2),
@@ -623,6 +666,14 @@ int ppk_hydro_create(const ppk_mhd_params *params, ppk_hydro_t **handle) {
   if (!h) return hfail(nullptr, PPK_ERR_OUT_OF_MEMORY, "host allocation failed");
   h->p = *params;
   h->hd = ppk::make_hydro_dev(*params);
+  // tuning knob, else the estimate
+  const char *strip = std::getenv("PPKMHD_HYDRO_STRIP");
+  const int rows = strip ? std::atoi(strip) : 0;
+  int dev = 0, cus = 0;
+  if (hipGetDevice(&dev) != hipSuccess ||
+      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
+    cus = 0;
+  h->hd.strip_rows = rows > 0 ? rows : ppk::hydro_strip_rows(h->hd, cus);
   const bool strict = params->precision == PPK_FP64_STRICT;
   h->K = strict ? &ppk::kStrict : &ppk::kFast;
   h->H = strict ? &ppk::kHydroStrict : &ppk::kHydroFast;
