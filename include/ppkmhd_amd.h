@@ -52,7 +52,8 @@ enum ppk_bc { PPK_BC_UNDEFINED = 0, PPK_BC_DIRICHLET = 1, PPK_BC_NEUMANN = 2,
 enum ppk_precision { PPK_FP64 = 0, PPK_FP32_BULK = 1, PPK_FP64_STRICT = 2 };
 /* kernel organisation of the step */
 enum ppk_kernel_path {
-  PPK_PATH_AUTO = 0,   /* fused kernels where available, else staged                         */
+  PPK_PATH_AUTO = 0,   /* fused kernels where available, else staged; of the fused forms the
+                        * one that is faster at the grid's size                              */
   PPK_PATH_STAGED = 1, /* one kernel per reference stage, intermediates in HBM                */
   PPK_PATH_FUSED = 2,  /* fused kernels: in FP64 the single-pass step (state read once and   
                         * written once), else the three-kernel form                          */

@@ -386,8 +386,8 @@ int ppk_mhd_create(const ppk_mhd_params *params, ppk_mhd_t **handle) {
   h->K = params->precision == PPK_FP64_STRICT ? &ppk::kStrict : &ppk::kFast;
   h->dp.bulk32 = params->precision == PPK_FP32_BULK ? 1 : 0;
   h->fused = ppk::fused_supported(h->dp, params->precision, params->kernel_path);
-  // FP64: the single-pass kernels, unless the three-kernel form is asked for (the FP32-bulk
-  // form and the surrogate run the three-kernel form)
+  // FP64: the single-pass kernels, unless the three-kernel form is asked for or is the faster
+  // one (the FP32-bulk form and the surrogate run the three-kernel form)
   int dev = 0, cus = 0;
   if (hipGetDevice(&dev) != hipSuccess ||
       hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
@@ -395,7 +395,9 @@ int ppk_mhd_create(const ppk_mhd_params *params, ppk_mhd_t **handle) {
   if (h->fused && params->precision != PPK_FP32_BULK &&
       params->kernel_path != PPK_PATH_FUSED_RECORDS) {
     if (params->dim == 3)
-      h->dp.march = ppk::march_nblk(h->dp, cus);
+      h->dp.march = params->kernel_path == PPK_PATH_FUSED || ppk::march_pays(h->dp, cus)
+                        ? ppk::march_nblk(h->dp, cus)
+                        : 0;
     else
       ppk::march2d_shape(h->dp, cus);
   }

@@ -162,15 +162,30 @@ inline Brick sub_bricks(const DevParams &p) {
 // The single-pass 3D step (march3d.hip): blocks of 16 x 12 output columns marching along z
 // through equal shares of the grid's tile-planes; one CFL partial per block
 constexpr int kMarchOutX = 16, kMarchOutY = 12;
-// Blocks of the launch: one per CU (each block needs a whole CU's LDS), fewer when a block
-// would get under 16 tile-planes (small grids)
+// Blocks of the launch: one per CU (each block needs a whole CU's LDS), fewer only when there
+// are fewer tile-planes.  Every segment starts with the work of about two planes more, but a CU
+// without a block gains nothing: at least 16 tile-planes per block left 231 CUs idle on a
+// 37 x 29 x 45 box (286 us per step, now 75).
 inline int march_nblk(const DevParams &p, int cus) {
   const long long total =
       (long long)((p.nx + kMarchOutX - 1) / kMarchOutX) * ((p.ny + kMarchOutY - 1) / kMarchOutY) *
       p.nz;
   long long b = cus > 0 ? cus : 256;
-  if (b > total / 16) b = total / 16;
+  if (b > total) b = total;
   return (int)(b < 1 ? 1 : b);
+}
+// PPK_PATH_AUTO: whether the single-pass 3D step is the faster form.  Its time is that of the
+// tile-planes of one block, 15 us each, two more per segment (a second segment where the ranges
+// cut tiles); the three-kernel form takes 0.43 us per 1000 cells once its launches are paid.
+// Measured us per step, single-pass / three-kernel: 16^3 44 / 32, 32^3 47 / 43, 37x29x45 75 / 47,
+// 48^3 79 / 76, 64^3 141 / 132, 80^3 212 / 248, 96^3 309 / 404, 160x20x20 62 / 62.
+inline bool march_pays(const DevParams &p, int cus) {
+  const double tiles =
+      (double)((p.nx + kMarchOutX - 1) / kMarchOutX) * ((p.ny + kMarchOutY - 1) / kMarchOutY);
+  const int b = march_nblk(p, cus);
+  const int planes = (int)((tiles * p.nz + b - 1) / b);
+  const double march = 28.0 + 15.2 * planes + (p.nz % planes ? 16.0 : 0.0);
+  return march < 27.0 + 0.43e-3 * p.nx * p.ny * (double)p.nz;
 }
 // The single-pass 2D step (march2d.hip): strips of lw - 4 output columns (lw = 64 or 32 lanes)
 // by `rows` output rows, 64 / lw strips per wave; one CFL partial per wave
