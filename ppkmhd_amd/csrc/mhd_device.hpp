@@ -76,6 +76,15 @@ constexpr bool kSharedRecip = false;
 #else
 constexpr bool kSharedRecip = true;
 #endif
+// The default build's solvers (kLean) take forms that need fewer square roots and quotients
+// than the reference's expressions; each such place says which.  PPK_KEEP_ROUNDING (the batched
+// kernels) leaves them out: a long ensemble amplifies last-bit differences of a step until two
+// builds of the library disagree in 11 digits, and ensembles are kept to be compared.
+#ifdef PPK_KEEP_ROUNDING
+constexpr bool kLean = false;
+#else
+constexpr bool kLean = kSharedRecip;
+#endif
 #if defined(__HIP_DEVICE_COMPILE__) && !defined(PPK_EXACT_DIV)
 // one third-order step from the hardware estimate r0 (relative error eps): with
 // e = 1 - b r0, 1/b = r0 (1 + e + e^2 + ...); with e = 1 - x y0^2, 1/sqrt(x) =
@@ -171,9 +180,23 @@ PPK_HD R max5(R a0, R a1, R a2, R a3, R a4) {
   return r;
 }
 
-// fast magnetosonic speed along dir, reference src/shared/mhd_utils.h:89-117
+// 1/a and 1/b from one reciprocal (neither may be zero or infinite): a product's rounding more
+// than two reciprocals, 10 instead of 14 issue slots on the GPU
 template <class R>
-PPK_HD R speed_fast(const St<R> &q, int dir, R gamma0) {
+PPK_HD void recip2(R a, R b, R &ia, R &ib) {
+  if (kLean) {
+    const R i = recip(a * b);
+    ia = b * i;
+    ib = a * i;
+  } else {
+    ia = recip(a);
+    ib = recip(b);
+  }
+}
+
+// square of the fast magnetosonic speed along dir, reference src/shared/mhd_utils.h:89-117
+template <class R>
+PPK_HD R speed_fast_sq(const St<R> &q, int dir, R gamma0) {
   R d = q[ID], p = q[IP], a = q[IA], b = q[IB], c = q[IC];
   const R id = recip(d);
   R b2 = a * a + b * b + c * c;
@@ -182,7 +205,28 @@ PPK_HD R speed_fast(const St<R> &q, int dir, R gamma0) {
   R bn = dir == IX ? a : (dir == IY ? b : c);
   // c2 bn^2 / d: in the default builds (c2 / d) bn^2, c2 / d shared by the directions of a state
   const R cbd = kSharedRecip ? (c2 * id) * (bn * bn) : c2 * bn * bn / d;
-  return msqrt(d2 + msqrt(nonneg(d2 * d2 - cbd)));
+  return d2 + msqrt(nonneg(d2 * d2 - cbd));
+}
+template <class R>
+PPK_HD R speed_fast(const St<R> &q, int dir, R gamma0) {
+  return msqrt(speed_fast_sq(q, dir, gamma0));
+}
+// the larger fast speed of two states along x; in the default builds the root of the larger
+// square (the same value: the square root is correctly rounded, hence monotone)
+template <class R>
+PPK_HD R max_speed_fast(const St<R> &l, const St<R> &r, R gamma0) {
+  if (kLean) return msqrt(dmax(speed_fast_sq(l, IX, gamma0), speed_fast_sq(r, IX, gamma0)));
+  return dmax(speed_fast(l, IX, gamma0), speed_fast(r, IX, gamma0));
+}
+// the largest of four states along dir, likewise
+template <class R>
+PPK_HD R max_speed_fast4(const St<R> &a, const St<R> &b, const St<R> &c, const St<R> &d, int dir,
+                         R gamma0) {
+  if (kLean)
+    return msqrt(max4(speed_fast_sq(a, dir, gamma0), speed_fast_sq(b, dir, gamma0),
+                      speed_fast_sq(c, dir, gamma0), speed_fast_sq(d, dir, gamma0)));
+  return max4(speed_fast(a, dir, gamma0), speed_fast(b, dir, gamma0), speed_fast(c, dir, gamma0),
+              speed_fast(d, dir, gamma0));
 }
 
 // per-cell CFL term sum_d (c_f,d + |v_d|)/dx_d, reference src/shared/mhd_utils.h:319-366 and
@@ -244,8 +288,14 @@ PPK_HD void constoprim(const St<R> &u, R magx, R magy, R magz, St<R> &q,
 // reference src/muscl/MHDBaseFunctor2D.h:308-327.  The default builds give the magnitude
 // the sign of dcen with copysign (one instruction for the compare, select and multiply by
 // +-1); the value is the same, only a zero slope at dcen = -0 keeps the sign of dcen.
+// The default solvers' minmod (kLean, a factor of 1 known at compile time) is the smaller of the
+// two differences where their signs agree: the central one, their mean, is never smaller.
 template <class R>
 PPK_HD R limited_slope(R st, R q, R qplus, R qminus) {
+  if (kLean && __builtin_constant_p(st) && st == R(1)) {
+    const R l = q - qminus, r = qplus - q;
+    return dmax(dmin(l, r), R(0)) + dmin(dmax(l, r), R(0));
+  }
   R dlft = st * (q - qminus);
   R drgt = st * (qplus - q);
   R dcen = R(0.5) * (qplus - qminus);
@@ -293,11 +343,9 @@ PPK_HD void riemann_hlld(St<R> &qleft, St<R> &qright, St<R> &flux,
   R ptotr = pr + emagr;
   R vdotbr = ur * a + vr * br + wr * cr;
 
-  R cfastl = speed_fast(qleft, IX, gamma0);
-  R cfastr = speed_fast(qright, IX, gamma0);
-
-  R sl = dmin(ul, ur) - dmax(cfastl, cfastr);
-  R sr = dmax(ul, ur) + dmax(cfastl, cfastr);
+  const R cfast = max_speed_fast(qleft, qright, gamma0);
+  R sl = dmin(ul, ur) - cfast;
+  R sr = dmax(ul, ur) + cfast;
 
   R rcl = rl * (ul - sl);
   R rcr = rr * (sr - ur);
@@ -312,7 +360,8 @@ PPK_HD void riemann_hlld(St<R> &qleft, St<R> &qright, St<R> &flux,
     return a * a > R(0) && (kSharedRecip ? dabs(estar - a * a) <= R(1e-8) * (a * a)
                                          : dabs(estar / (a * a) - R(1)) <= R(1e-8));
   };
-  const R isl = recip(sl - ustar);
+  R isl, isr;
+  recip2(sl - ustar, sr - ustar, isl, isr);
   R rstarl = divr(rl * (sl - ul), sl - ustar, isl);
   R estar = rl * (sl - ul) * (sl - ustar) - a * a;
   R el = rl * (sl - ul) * (sl - ul) - a * a;
@@ -322,6 +371,12 @@ PPK_HD void riemann_hlld(St<R> &qleft, St<R> &qright, St<R> &flux,
     bstarl = bl;
     wstarl = wl;
     cstarl = cl;
+  } else if (kLean) {  // the common factors of the four values first
+    const R ie = recip(estar), f = a * (ustar - ul) * ie, g = el * ie;
+    vstarl = vl - bl * f;
+    bstarl = bl * g;
+    wstarl = wl - cl * f;
+    cstarl = cl * g;
   } else {
     const R ie = recip(estar);
     vstarl = vl - divr(a * bl * (ustar - ul), estar, ie);
@@ -333,10 +388,10 @@ PPK_HD void riemann_hlld(St<R> &qleft, St<R> &qright, St<R> &flux,
   R etotstarl = divr((sl - ul) * etotl - ptotl * ul + ptotstar * ustar + a * (vdotbl - vdotbstarl),
                      sl - ustar, isl);
   R sqrrstarl = msqrt(rstarl);
-  R calfvenl = over_sqrt(dabs(a), rstarl);
-  R sal = ustar - calfvenl;
+  // only the signs of the Alfven wave speeds u* -+ |a| / sqrt(rho*) are used; sqrt(rho*) > 0
+  // times the speed has the same sign and needs no quotient
+  R sal = kLean ? ustar * sqrrstarl - dabs(a) : ustar - over_sqrt(dabs(a), rstarl);
 
-  const R isr = recip(sr - ustar);
   R rstarr = divr(rr * (sr - ur), sr - ustar, isr);
   estar = rr * (sr - ur) * (sr - ustar) - a * a;
   R er = rr * (sr - ur) * (sr - ur) - a * a;
@@ -346,6 +401,12 @@ PPK_HD void riemann_hlld(St<R> &qleft, St<R> &qright, St<R> &flux,
     bstarr = br;
     wstarr = wr;
     cstarr = cr;
+  } else if (kLean) {
+    const R ie = recip(estar), f = a * (ustar - ur) * ie, g = er * ie;
+    vstarr = vr - br * f;
+    bstarr = br * g;
+    wstarr = wr - cr * f;
+    cstarr = cr * g;
   } else {
     const R ie = recip(estar);
     vstarr = vr - divr(a * br * (ustar - ur), estar, ie);
@@ -357,8 +418,7 @@ PPK_HD void riemann_hlld(St<R> &qleft, St<R> &qright, St<R> &flux,
   R etotstarr = divr((sr - ur) * etotr - ptotr * ur + ptotstar * ustar + a * (vdotbr - vdotbstarr),
                      sr - ustar, isr);
   R sqrrstarr = msqrt(rstarr);
-  R calfvenr = over_sqrt(dabs(a), rstarr);
-  R sar = ustar + calfvenr;
+  R sar = kLean ? ustar * sqrrstarr + dabs(a) : ustar + over_sqrt(dabs(a), rstarr);
 
   const R isq = recip(sqrrstarl + sqrrstarr);
   R vstarstar = divr(sqrrstarl * vstarl + sqrrstarr * vstarr + sgnm * (bstarr - bstarl),
@@ -441,10 +501,9 @@ PPK_HD void riemann_hll(St<R> &ql, St<R> &qr, St<R> &flux,
   St<R> ul, fl, ur, fr;
   mhd_flux(ql, ul, fl, par);
   mhd_flux(qr, ur, fr, par);
-  R cfl = speed_fast(ql, IX, R(par.gamma0));
-  R cfr = speed_fast(qr, IX, R(par.gamma0));
-  R sl = dmin(dmin(ql[IU], qr[IU]) - dmax(cfl, cfr), R(0));
-  R sr = dmax(dmax(ql[IU], qr[IU]) + dmax(cfl, cfr), R(0));
+  const R cf = max_speed_fast(ql, qr, R(par.gamma0));
+  R sl = dmin(dmin(ql[IU], qr[IU]) - cf, R(0));
+  R sr = dmax(dmax(ql[IU], qr[IU]) + cf, R(0));
 #pragma unroll
   for (int v = 0; v < 8; ++v)
     flux[v] = (sr * fl[v] - sl * fr[v] + sr * sl * (ur[v] - ul[v])) / (sr - sl);
@@ -514,19 +573,12 @@ PPK_HD R mag_riemann2d_hlld(const St<R> &qLL, const St<R> &qRL,
   R rRL = qRL[ID], pRL = qRL[IP], uRL = qRL[IU], vRL = qRL[IV], aRL = qRL[IA], bRL = qRL[IB], cRL = qRL[IC];
   R rRR = qRR[ID], pRR = qRR[IP], uRR = qRR[IU], vRR = qRR[IV], aRR = qRR[IA], bRR = qRR[IB], cRR = qRR[IC];
 
-  R cFastLLx = speed_fast(qLL, IX, gamma0);
-  R cFastLRx = speed_fast(qLR, IX, gamma0);
-  R cFastRLx = speed_fast(qRL, IX, gamma0);
-  R cFastRRx = speed_fast(qRR, IX, gamma0);
-  R cFastLLy = speed_fast(qLL, IY, gamma0);
-  R cFastLRy = speed_fast(qLR, IY, gamma0);
-  R cFastRLy = speed_fast(qRL, IY, gamma0);
-  R cFastRRy = speed_fast(qRR, IY, gamma0);
-
-  R SL = min4(uLL, uLR, uRL, uRR) - max4(cFastLLx, cFastLRx, cFastRLx, cFastRRx);
-  R SR = max4(uLL, uLR, uRL, uRR) + max4(cFastLLx, cFastLRx, cFastRLx, cFastRRx);
-  R SB = min4(vLL, vLR, vRL, vRR) - max4(cFastLLy, cFastLRy, cFastRLy, cFastRRy);
-  R ST = max4(vLL, vLR, vRL, vRR) + max4(cFastLLy, cFastLRy, cFastRLy, cFastRRy);
+  const R cx = max_speed_fast4(qLL, qLR, qRL, qRR, IX, gamma0);
+  const R cy = max_speed_fast4(qLL, qLR, qRL, qRR, IY, gamma0);
+  R SL = min4(uLL, uLR, uRL, uRR) - cx;
+  R SR = max4(uLL, uLR, uRL, uRR) + cx;
+  R SB = min4(vLL, vLR, vRL, vRR) - cy;
+  R ST = max4(vLL, vLR, vRL, vRR) + cy;
 
   R PtotLL = pLL + R(0.5) * (aLL * aLL + bLL * bLL + cLL * cLL);
   R PtotLR = pLR + R(0.5) * (aLR * aLR + bLR * bLR + cLR * cLR);
@@ -543,68 +595,105 @@ PPK_HD R mag_riemann2d_hlld(const St<R> &qLL, const St<R> &qRL,
   R rcRRy = rRR * (ST - vRR);
 
   const R rcx = rcLLx + rcLRx + rcRLx + rcRRx, rcy = rcLLy + rcLRy + rcRLy + rcRRy;
+  R ircx, ircy;
+  recip2(rcx, rcy, ircx, ircy);
   R ustar = divr(rcLLx * uLL + rcLRx * uLR + rcRLx * uRL + rcRRx * uRR +
                      (PtotLL - PtotRL + PtotLR - PtotRR),
-                 rcx, recip(rcx));
+                 rcx, ircx);
   R vstar = divr(rcLLy * vLL + rcLRy * vLR + rcRLy * vRL + rcRRy * vRR +
                      (PtotLL - PtotLR + PtotRL - PtotRR),
-                 rcy, recip(rcy));
+                 rcy, ircy);
 
-  const R iSLu = recip(SL - ustar), iSRu = recip(SR - ustar);
-  const R iSBv = recip(SB - vstar), iSTv = recip(ST - vstar);
+  R iSLu, iSRu, iSBv, iSTv;
+  recip2(SL - ustar, SR - ustar, iSLu, iSRu);
+  recip2(SB - vstar, ST - vstar, iSBv, iSTv);
 
   R rstarLLx = divr(rLL * (SL - uLL), SL - ustar, iSLu);
-  R BstarLL = divr(bLL * (SL - uLL), SL - ustar, iSLu);
+  R BstarLL = kLean ? bLL * ((SL - uLL) * iSLu)
+                   : divr(bLL * (SL - uLL), SL - ustar, iSLu);
   R rstarLLy = divr(rLL * (SB - vLL), SB - vstar, iSBv);
-  R AstarLL = divr(aLL * (SB - vLL), SB - vstar, iSBv);
+  R AstarLL = kLean ? aLL * ((SB - vLL) * iSBv)
+                   : divr(aLL * (SB - vLL), SB - vstar, iSBv);
   R rstarLL = divr(divr(rLL * (SL - uLL), SL - ustar, iSLu) * (SB - vLL), SB - vstar, iSBv);
   R EstarLLx = ustar * BstarLL - vLL * aLL;
   R EstarLLy = uLL * bLL - vstar * AstarLL;
   R EstarLL = ustar * BstarLL - vstar * AstarLL;
 
   R rstarLRx = divr(rLR * (SL - uLR), SL - ustar, iSLu);
-  R BstarLR = divr(bLR * (SL - uLR), SL - ustar, iSLu);
+  R BstarLR = kLean ? bLR * ((SL - uLR) * iSLu)
+                   : divr(bLR * (SL - uLR), SL - ustar, iSLu);
   R rstarLRy = divr(rLR * (ST - vLR), ST - vstar, iSTv);
-  R AstarLR = divr(aLR * (ST - vLR), ST - vstar, iSTv);
+  R AstarLR = kLean ? aLR * ((ST - vLR) * iSTv)
+                   : divr(aLR * (ST - vLR), ST - vstar, iSTv);
   R rstarLR = divr(divr(rLR * (SL - uLR), SL - ustar, iSLu) * (ST - vLR), ST - vstar, iSTv);
   R EstarLRx = ustar * BstarLR - vLR * aLR;
   R EstarLRy = uLR * bLR - vstar * AstarLR;
   R EstarLR = ustar * BstarLR - vstar * AstarLR;
 
   R rstarRLx = divr(rRL * (SR - uRL), SR - ustar, iSRu);
-  R BstarRL = divr(bRL * (SR - uRL), SR - ustar, iSRu);
+  R BstarRL = kLean ? bRL * ((SR - uRL) * iSRu)
+                   : divr(bRL * (SR - uRL), SR - ustar, iSRu);
   R rstarRLy = divr(rRL * (SB - vRL), SB - vstar, iSBv);
-  R AstarRL = divr(aRL * (SB - vRL), SB - vstar, iSBv);
+  R AstarRL = kLean ? aRL * ((SB - vRL) * iSBv)
+                   : divr(aRL * (SB - vRL), SB - vstar, iSBv);
   R rstarRL = divr(divr(rRL * (SR - uRL), SR - ustar, iSRu) * (SB - vRL), SB - vstar, iSBv);
   R EstarRLx = ustar * BstarRL - vRL * aRL;
   R EstarRLy = uRL * bRL - vstar * AstarRL;
   R EstarRL = ustar * BstarRL - vstar * AstarRL;
 
   R rstarRRx = divr(rRR * (SR - uRR), SR - ustar, iSRu);
-  R BstarRR = divr(bRR * (SR - uRR), SR - ustar, iSRu);
+  R BstarRR = kLean ? bRR * ((SR - uRR) * iSRu)
+                   : divr(bRR * (SR - uRR), SR - ustar, iSRu);
   R rstarRRy = divr(rRR * (ST - vRR), ST - vstar, iSTv);
-  R AstarRR = divr(aRR * (ST - vRR), ST - vstar, iSTv);
+  R AstarRR = kLean ? aRR * ((ST - vRR) * iSTv)
+                   : divr(aRR * (ST - vRR), ST - vstar, iSTv);
   R rstarRR = divr(divr(rRR * (SR - uRR), SR - ustar, iSRu) * (ST - vRR), ST - vstar, iSTv);
   R EstarRRx = ustar * BstarRR - vRR * aRR;
   R EstarRRy = uRR * bRR - vstar * AstarRR;
   R EstarRR = ustar * BstarRR - vstar * AstarRR;
 
   const R smallc = R(p.smallc);
-  R calfvenL = max5(over_sqrt(dabs(aLR), rstarLRx), over_sqrt(dabs(AstarLR), rstarLR),
-                    over_sqrt(dabs(aLL), rstarLLx), over_sqrt(dabs(AstarLL), rstarLL), smallc);
-  R calfvenR = max5(over_sqrt(dabs(aRR), rstarRRx), over_sqrt(dabs(AstarRR), rstarRR),
-                    over_sqrt(dabs(aRL), rstarRLx), over_sqrt(dabs(AstarRL), rstarRL), smallc);
-  R calfvenB = max5(over_sqrt(dabs(bLL), rstarLLy), over_sqrt(dabs(BstarLL), rstarLL),
-                    over_sqrt(dabs(bRL), rstarRLy), over_sqrt(dabs(BstarRL), rstarRL), smallc);
-  R calfvenT = max5(over_sqrt(dabs(bLR), rstarLRy), over_sqrt(dabs(BstarLR), rstarLR),
-                    over_sqrt(dabs(bRR), rstarRRy), over_sqrt(dabs(BstarRR), rstarRR), smallc);
-
+  R calfvenL, calfvenR, calfvenB, calfvenT;
+  if (kLean) {
+    // The larger of |A| / sqrt(rho*_x) and |A*| / sqrt(rho*), with rho*_x = rho fx, A* = A fy and
+    // rho* = rho fx fy, is the root of A^2 max(1, fy) / (rho fx); of two states the larger
+    // fraction is found by cross multiplication, and sqrt(n / d) = n rsq(n d): one inverse
+    // square root per side instead of four.  n = 0 gives a NaN, which the maximum drops.
+    const auto alfven = [&](R n1, R d1, R n2, R d2) {
+      const bool first = n1 * d2 > n2 * d1;
+      const R n = first ? n1 : n2, d = first ? d1 : d2;
+      return dmax(over_sqrt(n, n * d), smallc);
+    };
+    const R one = R(1);
+    const R fxLL = (SL - uLL) * iSLu, fxLR = (SL - uLR) * iSLu;
+    const R fxRL = (SR - uRL) * iSRu, fxRR = (SR - uRR) * iSRu;
+    const R fyLL = (SB - vLL) * iSBv, fyRL = (SB - vRL) * iSBv;
+    const R fyLR = (ST - vLR) * iSTv, fyRR = (ST - vRR) * iSTv;
+    calfvenL = alfven(aLR * aLR * dmax(one, fyLR), rLR * fxLR, aLL * aLL * dmax(one, fyLL),
+                      rLL * fxLL);
+    calfvenR = alfven(aRR * aRR * dmax(one, fyRR), rRR * fxRR, aRL * aRL * dmax(one, fyRL),
+                      rRL * fxRL);
+    calfvenB = alfven(bLL * bLL * dmax(one, fxLL), rLL * fyLL, bRL * bRL * dmax(one, fxRL),
+                      rRL * fyRL);
+    calfvenT = alfven(bLR * bLR * dmax(one, fxLR), rLR * fyLR, bRR * bRR * dmax(one, fxRR),
+                      rRR * fyRR);
+  } else {
+    calfvenL = max5(over_sqrt(dabs(aLR), rstarLRx), over_sqrt(dabs(AstarLR), rstarLR),
+                  over_sqrt(dabs(aLL), rstarLLx), over_sqrt(dabs(AstarLL), rstarLL), smallc);
+    calfvenR = max5(over_sqrt(dabs(aRR), rstarRRx), over_sqrt(dabs(AstarRR), rstarRR),
+                  over_sqrt(dabs(aRL), rstarRLx), over_sqrt(dabs(AstarRL), rstarRL), smallc);
+    calfvenB = max5(over_sqrt(dabs(bLL), rstarLLy), over_sqrt(dabs(BstarLL), rstarLL),
+                  over_sqrt(dabs(bRL), rstarRLy), over_sqrt(dabs(BstarRL), rstarRL), smallc);
+    calfvenT = max5(over_sqrt(dabs(bLR), rstarLRy), over_sqrt(dabs(BstarLR), rstarLR),
+                  over_sqrt(dabs(bRR), rstarRRy), over_sqrt(dabs(BstarRR), rstarRR), smallc);
+  }
   R SAL = dmin(ustar - calfvenL, R(0));
   R SAR = dmax(ustar + calfvenR, R(0));
   R SAB = dmin(vstar - calfvenB, R(0));
   R SAT = dmax(vstar + calfvenT, R(0));
 
-  const R iSAx = recip(SAR - SAL), iSAy = recip(SAT - SAB);
+  R iSAx, iSAy;
+  recip2(SAR - SAL, SAT - SAB, iSAx, iSAy);
   R AstarT = divr(SAR * AstarRR - SAL * AstarLR, SAR - SAL, iSAx);
   R AstarB = divr(SAR * AstarRL - SAL * AstarLL, SAR - SAL, iSAx);
   R BstarR = divr(SAT * BstarRR - SAB * BstarRL, SAT - SAB, iSAy);
