@@ -181,6 +181,10 @@ struct MarchThread {
   double pq[2][11], pf[2][3];
   bool pqok[2], pfok[2];
   double cfl;        // maximum CFL term of this thread's output cells (over every segment)
+  // byte offsets within a plane of its Q and face cells and of its column (a plane of a grid of
+  // 2^31 cells and at least 9 planes has under 2^28): each access is a uniform base plus one of
+  // them, where 64-bit cell indices took two or three instructions per access
+  unsigned oq[2], of[2], oc;
 
   PPK_HD void init(const DevParams &p, int t, int x0, int y0) {
     tid = t;
@@ -193,34 +197,55 @@ struct MarchThread {
     ocol = t < kMC && a >= 1 && a <= kMOX && b >= 1 && b <= kMOY && in;
     acol = rok && a >= 1 && b >= 1 && b <= kMOY && j < p.jsize - p.gw;
     bcol = rok && b >= 1 && a >= 1 && a <= kMOX && i < p.isize - p.gw;
+    const int qhi = 1 - p.gw;  // Q cells up to size + qhi (the reference's primitive range)
+#pragma unroll
+    for (int it = 0; it < 2; ++it) {
+      const int n = t + it * kMN;
+      int ii = x0 - 1 + n % kQW, jj = y0 - 1 + n / kQW;
+      pqok[it] = n < kQN && ii <= p.isize + qhi && jj <= p.jsize + qhi;
+      oq[it] = offset(p, min(ii, p.isize + qhi), min(jj, p.jsize + qhi));
+      ii = x0 - 1 + n % kFW;
+      jj = y0 - 1 + n / kFW;
+      pfok[it] = n < kFN && ii < p.isize && jj < p.jsize;
+      of[it] = offset(p, min(ii, p.isize - 1), min(jj, p.jsize - 1));
+    }
+    oc = offset(p, min(i, p.isize - 1), min(j, p.jsize - 1));
+  }
+  PPK_HD static unsigned offset(const DevParams &p, int ii, int jj) {
+    return 8u * ((unsigned)jj * (unsigned)p.isize + (unsigned)ii);
+  }
+  // An offset at the place of its loads.  It is made opaque there: widened to 64 bits outside the
+  // loop, it would cost a 64-bit vector addition per load instead of a load from a scalar base.
+  PPK_HD static unsigned here(unsigned byte) {
+#ifdef __HIP_DEVICE_COMPILE__
+    asm volatile("" : "+v"(byte));
+#endif
+    return byte;
+  }
+  PPK_HD static double at(const double *__restrict__ base, unsigned byte) {
+    return *reinterpret_cast<const double *>(reinterpret_cast<const char *>(base) + byte);
   }
 
   // global loads of plane pl for its Q and face cells (issued early, stashed later)
   PPK_HD void prefetch(const double *__restrict__ U, const DevParams &p, int x0, int y0,
                        int pl) {
     const long long vs = p.vstride;
-    const int qhi = 1 - p.gw;  // Q cells up to size + qhi (the reference's primitive range)
+    const double *base = U + (long long)pl * p.plane;
 #pragma unroll
     for (int it = 0; it < 2; ++it) {
-      const int n = tid + it * kMN;
-      const int ii = x0 - 1 + n % kQW, jj = y0 - 1 + n / kQW;
-      pqok[it] = n < kQN && ii <= p.isize + qhi && jj <= p.jsize + qhi;
-      const long long t = cidx(p, min(ii, p.isize + qhi), min(jj, p.jsize + qhi), pl);
+      const unsigned o = here(oq[it]);
 #pragma unroll
-      for (int v = 0; v < 8; ++v) pq[it][v] = U[t + v * vs];
-      pq[it][8] = U[t + 1 + IA * vs];
-      pq[it][9] = U[t + p.isize + IB * vs];
-      pq[it][10] = U[t + p.plane + IC * vs];
+      for (int v = 0; v < 8; ++v) pq[it][v] = at(base + v * vs, o);
+      pq[it][8] = at(base + IA * vs + 1, o);
+      pq[it][9] = at(base + IB * vs + p.isize, o);
+      pq[it][10] = at(base + IC * vs + p.plane, o);
     }
 #pragma unroll
     for (int it = 0; it < 2; ++it) {
-      const int n = tid + it * kMN;
-      const int ii = x0 - 1 + n % kFW, jj = y0 - 1 + n / kFW;
-      pfok[it] = n < kFN && ii < p.isize && jj < p.jsize;
-      const long long t = cidx(p, min(ii, p.isize - 1), min(jj, p.jsize - 1), pl);
-      pf[it][0] = U[t + IA * vs];
-      pf[it][1] = U[t + IB * vs];
-      pf[it][2] = U[t + IC * vs];
+      const unsigned o = here(of[it]);
+      pf[it][0] = at(base + IA * vs, o);
+      pf[it][1] = at(base + IB * vs, o);
+      pf[it][2] = at(base + IC * vs, o);
     }
   }
 
@@ -301,9 +326,10 @@ struct MarchThread {
   // the state of plane r that the update starts from (issued early)
   PPK_HD void load_state(const double *__restrict__ U, const DevParams &p, int r) {
     if (!(rok && a >= 1 && b >= 1)) return;
-    const long long t = cidx(p, i, j, r);
+    const double *base = U + (long long)r * p.plane;
+    const unsigned o = here(oc);
 #pragma unroll
-    for (int v = 0; v < 8; ++v) Uc[v] = U[t + v * p.vstride];
+    for (int v = 0; v < 8; ++v) Uc[v] = at(base + v * p.vstride, o);
   }
 
   // H(r): the record of the column at plane r (slot sa: plane r, slot sb: plane r+1), same
@@ -471,9 +497,11 @@ struct MarchThread {
         un[IA] = Ap - (ey - Eym) * dtdz;
         un[IB] = Bp + (ex - Exm) * dtdz;
         un[IC] = Cf;
-        const long long t = cidx(p, i, j, r - 1);
+        char *base = reinterpret_cast<char *>(Uout + (long long)(r - 1) * p.plane);
+        const unsigned o = here(oc);
 #pragma unroll
-        for (int v = 0; v < 8; ++v) Uout[t + v * p.vstride] = un[v];
+        for (int v = 0; v < 8; ++v)
+          *reinterpret_cast<double *>(base + 8 * v * p.vstride + o) = un[v];
       }
       if (fold) {
         if (acol) sC[tid] = Ap - (ey - Eym) * dtdz;
