@@ -140,17 +140,21 @@ HydroDev make_hydro_dev(const ppk_mhd_params &p) {
 // The estimates are in us per row or plane; measured per step (MI355X, HLLC, best in brackets):
 //   2D  64^2     64 rows 114, 8 rows 23, [1 row 12]
 //       1024^2   64 rows 116, [6 rows 44], 12 rows 46, 1 row 69
-//       4096x2048  128 rows 365, 64 rows 270, [20 rows 225], 47 rows 227
+//       4096x2048  128 rows 360, 64 rows 249, 40 rows 220, [24 rows 207], 16 rows 216
+//       6000x3000  96 rows 479, 64 rows 429, 40 rows 435, [24 rows 419], 16 rows 428
+//       8192x4096  128 rows 820, 64 rows 767, [40 rows 763], 24 rows 768, 16 rows 782
 //   3D  64^3     48 planes 252, 8 planes 58, [4 planes 41], 1 plane 63
 //       256x192x128  48 planes 454, [64 planes 381], 16 planes 400, 1 plane 866
-// (48 planes and 64 rows were the fixed values.)
+// (48 planes and 64 rows were the fixed values.)  In 2D more than 24 rows never gain more than 1 %
+// and can lose 10 % to a last round that is nearly empty.
 int hydro_strip_rows(const HydroDev &d, int cus) {
   if (cus <= 0) cus = 256;
   const int n = d.dim == 3 ? d.nz : d.ny;
   const auto up = [](double a, double b) { return std::ceil(a / b); };
   int pick = 1;
   double best = 0.0;
-  for (int r = 1; r <= n; ++r) {
+  const int most = d.dim == 3 ? n : std::min(n, 24);
+  for (int r = 1; r <= most; ++r) {
     double t;
     if (d.dim == 2) {
       // one wave per SIMD takes 1.6 us a row, more share its issue slots (1.35 to 1.4 each)
