@@ -49,77 +49,74 @@ PPK_HD void store(R *flux, const DevParams &p, long long c, const St<R> &f) {
     store_flux2<D>(flux, p, c, f);
 }
 
-// the faces of direction D of the bricks this block walks (see k_face_sur); w: the network in
-// LDS, sX: this wave's LDS slice; counts of faces by the network / in total accumulate
+// the faces of direction D of cell c (< 0: none; see k_face_sur); w: the network in LDS, sX: this
+// wave's LDS slice; counts of faces by the network / in total accumulate
 template <int DIM, int D, class R>
 __device__ __forceinline__ void faces_dir(const R *__restrict__ rec, R *__restrict__ flux,
-                                          const DevParams &p, const Brick &bk,
+                                          const DevParams &p, long long c,
                                           const SurrogateCfg &cfg, const MlpView &w,
                                           uint16_t *sX, unsigned long long &n_net,
                                           unsigned long long &n_all) {
   const int lane = lane_id();
   float *sY = reinterpret_cast<float *>(sX);
   const float gamma0 = float(p.gamma0);
-  const long long nb = bk.nblocks;
-#pragma unroll 1
-  for (long long L = blockIdx.x; L < nb; L += gridDim.x) {
-    const long long c = sub_brick_cell(p, bk, (int)L, threadIdx.x);
-    // the face states, the LLF pieces, the features and the check in float: their rounding
-    // is far below the network's own error; faces left to HLLD are recomputed in R there
-    St<float> a, b;
-    St<R> F;
-    bool gate = false;
-    if (c >= 0) {
-      states<DIM, D>(rec, p, c, a, b);
-      gate = smooth_face(a, b, cfg.gate_rho, cfg.gate_p);
-    }
-    bool use = false;
-    if (__ballot(gate) != 0ull) {  // the network runs for the whole wavefront (wave-uniform)
-      St<float> Fl;
-      float s = 1.f, rb = 1.f;
-      float x[kMlpIn];
-      if (gate) {
-        St<float> ul, ur, fl, fr;
-        llf_parts(a, b, ul, ur, fl, fr, s, Fl, p);
-        face_features(a, b, s, gamma0, x, rb);
-      } else {
-#pragma unroll
-        for (int i = 0; i < kMlpIn; ++i) x[i] = w.mu_in[i];
-      }
-#pragma unroll
-      for (int i = 0; i < kMlpIn; ++i)
-        sX[lane * 16 + i] = __builtin_bit_cast(uint16_t, bf16b((x[i] - w.mu_in[i]) * w.isig_in[i]));
-      wave_lds_sync();
-      mlp_infer_wave<kNB>(w, sX, sY);
-      if (gate) {
-        float sc[kMlpOut];
-        out_scales(rb, s, sc);
-        St<float> Fs, ul, ur, fl, fr;
-#pragma unroll
-        for (int o = 0; o < kMlpOut; ++o)
-          Fs[o] = Fl[o] + sc[o] * (w.mu_out[o] + w.sig_out[o] * sY[lane * 8 + o]);
-        mhd_flux(a, ul, fl, p);
-        mhd_flux(b, ur, fr, p);
-        use = admissible(ul, ur, fl, fr, Fs, s, gamma0);
-        if (use) {
-#pragma unroll
-          for (int o = 0; o < 8; ++o) F[o] = R(Fs[o]);
-        }
-      }
-    }
-    // the network's flux, or a mark for the HLLD pass (which keeps this kernel's registers
-    // free of the HLLD solver)
-    if (c >= 0) {
-      if (use) store<DIM, D>(flux, p, c, F);
-      cfg.flags[(long long)D * p.vstride + c] = use ? 0 : 1;
-    }
-    n_net += __popcll(__ballot(c >= 0 && use));
-    n_all += __popcll(__ballot(c >= 0));
+  // the face states, the LLF pieces, the features and the check in float: their rounding
+  // is far below the network's own error; faces left to HLLD are recomputed in R there
+  St<float> a, b;
+  St<R> F;
+  bool gate = false;
+  if (c >= 0) {
+    states<DIM, D>(rec, p, c, a, b);
+    gate = smooth_face(a, b, cfg.gate_rho, cfg.gate_p);
   }
+  bool use = false;
+  if (__ballot(gate) != 0ull) {  // the network runs for the whole wavefront (wave-uniform)
+    St<float> Fl;
+    float s = 1.f, rb = 1.f;
+    float x[kMlpIn];
+    if (gate) {
+      St<float> ul, ur, fl, fr;
+      llf_parts(a, b, ul, ur, fl, fr, s, Fl, p);
+      face_features(a, b, s, gamma0, x, rb);
+    } else {
+#pragma unroll
+      for (int i = 0; i < kMlpIn; ++i) x[i] = w.mu_in[i];
+    }
+#pragma unroll
+    for (int i = 0; i < kMlpIn; ++i)
+      sX[lane * 16 + i] = __builtin_bit_cast(uint16_t, bf16b((x[i] - w.mu_in[i]) * w.isig_in[i]));
+    wave_lds_sync();
+    mlp_infer_wave<kNB>(w, sX, sY);
+    if (gate) {
+      float sc[kMlpOut];
+      out_scales(rb, s, sc);
+      St<float> Fs, ul, ur, fl, fr;
+#pragma unroll
+      for (int o = 0; o < kMlpOut; ++o)
+        Fs[o] = Fl[o] + sc[o] * (w.mu_out[o] + w.sig_out[o] * sY[lane * 8 + o]);
+      mhd_flux(a, ul, fl, p);
+      mhd_flux(b, ur, fr, p);
+      use = admissible(ul, ur, fl, fr, Fs, s, gamma0);
+      if (use) {
+#pragma unroll
+        for (int o = 0; o < 8; ++o) F[o] = R(Fs[o]);
+      }
+    }
+  }
+  // the network's flux, or a mark for the HLLD pass (which keeps this kernel's registers
+  // free of the HLLD solver)
+  if (c >= 0) {
+    if (use) store<DIM, D>(flux, p, c, F);
+    cfg.flags[(long long)D * p.vstride + c] = use ? 0 : 1;
+  }
+  n_net += __popcll(__ballot(c >= 0 && use));
+  n_all += __popcll(__ballot(c >= 0));
 }
 
 // The learned face fluxes of every direction in one launch: a block stages the network in
-// LDS once and walks its bricks for direction x, then y (then z); see the file comment.
+// LDS once and walks its bricks, the directions of a brick one after another, so that its records
+// are read from the caches for all but the first (1024^2 133 -> 124 us a launch against all bricks
+// for x, then for y; 96^3 155 both ways); see the file comment.
 template <int DIM, class R>
 __global__ void __launch_bounds__(kBlock) k_face_sur(const R *__restrict__ rec,
                                                      R *__restrict__ flux, DevParams p, Brick bk,
@@ -155,9 +152,14 @@ __global__ void __launch_bounds__(kBlock) k_face_sur(const R *__restrict__ rec,
   const int wave = threadIdx.x >> 6, lane = lane_id();
   uint16_t *sX = sXall[wave];
   unsigned long long n_net = 0, n_all = 0;  // faces of this wave by the network, in total
-  faces_dir<DIM, 0, R>(rec, flux, p, bk, cfg, w, sX, n_net, n_all);
-  faces_dir<DIM, 1, R>(rec, flux, p, bk, cfg, w, sX, n_net, n_all);
-  if constexpr (DIM == 3) faces_dir<DIM, 2, R>(rec, flux, p, bk, cfg, w, sX, n_net, n_all);
+  const long long nb = bk.nblocks;
+#pragma unroll 1
+  for (long long L = blockIdx.x; L < nb; L += gridDim.x) {
+    const long long c = sub_brick_cell(p, bk, (int)L, threadIdx.x);
+    faces_dir<DIM, 0, R>(rec, flux, p, c, cfg, w, sX, n_net, n_all);
+    faces_dir<DIM, 1, R>(rec, flux, p, c, cfg, w, sX, n_net, n_all);
+    if constexpr (DIM == 3) faces_dir<DIM, 2, R>(rec, flux, p, c, cfg, w, sX, n_net, n_all);
+  }
   // per-block counts (no same-address atomics): this block's slots, in stream order
   if (cfg.counters) {
     __shared__ unsigned long long cnt[2][kBlock / 64];
