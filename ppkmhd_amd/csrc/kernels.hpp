@@ -37,7 +37,7 @@ enum Stage {
   ST_FUSED_RIEMANN,  // fused: Riemann problems at faces + EMFs at edges
   ST_FUSED_UPDATE,   // fused: update + CT + ghost copy (+ CFL of the new state)
   ST_FUSED_CFL,      // fused: standalone CFL reduction
-  ST_FUSED_MARCH,    // single-pass 3D step (half step, solves, update, CT, CFL in one kernel)
+  ST_FUSED_MARCH,    // single-pass step (half step, solves, update, CT, CFL in one kernel)
   ST_SUR_FACES,      // surrogate form: the network's face solves (inside ST_FUSED_RIEMANN)
   ST_SUR_FALLBACK,   // surrogate form: exact HLLD of the refused faces (same)
   ST_COUNT
@@ -165,7 +165,7 @@ constexpr int kMarchOutX = 16, kMarchOutY = 12;
 // Blocks of the launch: one per CU (each block needs a whole CU's LDS), fewer only when there
 // are fewer tile-planes.  Every segment starts with the work of about two planes more, but a CU
 // without a block gains nothing: at least 16 tile-planes per block left 231 CUs idle on a
-// 37 x 29 x 45 box (286 us per step, now 75).
+// 37 x 29 x 45 box (286 us per step, then 75).
 inline int march_nblk(const DevParams &p, int cus) {
   const long long total =
       (long long)((p.nx + kMarchOutX - 1) / kMarchOutX) * ((p.ny + kMarchOutY - 1) / kMarchOutY) *
@@ -177,8 +177,8 @@ inline int march_nblk(const DevParams &p, int cus) {
 // PPK_PATH_AUTO: whether the single-pass 3D step is the faster form.  Its time is that of the
 // tile-planes of one block, 15 us each, two more per segment (a second segment where the ranges
 // cut tiles); the three-kernel form takes 0.43 us per 1000 cells once its launches are paid.
-// Measured us per step, single-pass / three-kernel: 16^3 44 / 32, 32^3 47 / 43, 37x29x45 75 / 47,
-// 48^3 79 / 76, 64^3 141 / 132, 80^3 212 / 248, 96^3 309 / 404, 160x20x20 62 / 62.
+// Measured us per step, single-pass / three-kernel: 16^3 41 / 32, 32^3 45 / 42, 37x29x45 76 / 45,
+// 48^3 74 / 75, 64^3 133 / 130, 72^3 153 / 162, 80^3 194 / 242, 96^3 284 / 398, 160x20x20 57 / 60.
 inline bool march_pays(const DevParams &p, int cus) {
   const double tiles =
       (double)((p.nx + kMarchOutX - 1) / kMarchOutX) * ((p.ny + kMarchOutY - 1) / kMarchOutY);
@@ -197,7 +197,8 @@ inline long long march2d_waves(const DevParams &p, int lw, int rows) {
 // passes and a start of about one more.  One wave per SIMD issues instructions in 9 of 10
 // cycles, so a second wave on the same SIMD hides the start but little else: two take 1.9 times
 // as long as one, and so on per further wave.  Few rows give many waves but more passes per
-// row.  Measured (us per launch, MI355X, Orszag-Tang; strips of 64 columns):
+// row.  Measured (us per launch, MI355X, Orszag-Tang; strips of 64 columns; the leaner solvers
+// since took 10 to 13 % off each):
 //   64^2    1 row 17.7, 2 rows 22.8, 3 rows 27.8        (128, 64, 44 waves)
 //   256^2   1 row 27.4, 2 rows 24.3, 4 rows 34.1        (1280, 640, 320)
 //   1024^2  8 rows 130, 10 rows 108, 20 rows 121, 32 rows 179  (2304, 1854, 936, 576)

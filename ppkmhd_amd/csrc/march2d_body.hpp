@@ -52,7 +52,7 @@ __device__ __forceinline__ double from_right(double x) { return __shfl_down(x, 1
 // Fix a value in its register, as a value read from memory is: the compiler neither contracts
 // its product into the sums of its users nor keeps its operands alive for that.  Applied to the
 // values that the three-kernel form passes through LDS and HBM, it rounds nearly as that form
-// does and takes the spills of k_march2d from 17 to 6 registers (2048^2: 364 -> 337 us).
+// does and took the spills of k_march2d from 17 to 6 registers (2048^2: 364 -> 337 us).
 __device__ __forceinline__ void settle(double &x) { asm volatile("" : "+v"(x)); }
 __device__ __forceinline__ void settle(St<double> &s) {
 #pragma unroll

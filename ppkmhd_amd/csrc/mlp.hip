@@ -4,10 +4,11 @@
 //   k_train   one wavefront per 16 samples, 8 wavefronts per block: standardise, forward
 //             (MFMA), loss gradient, backward to the pre-activation gradients (MFMA with the
 //             transposed weights); the network and the bf16 activations and gradients of the
-//             block's 128 samples are in LDS, the latter feature-major, and the block sums its weight gradients dW = dZ^T H
-//             from there (MFMA, the samples are the k dimension); FP32 partials per block
-//   k_adam    sums the partials (FP64), applies Adam to the FP32 master parameters and refreshes the
-//             bf16 operand copies of each weight
+//             block's 128 samples are in LDS, the latter feature-major, and the block sums its
+//             weight gradients dW = dZ^T H from there (MFMA, the samples are the k dimension);
+//             FP32 partials per block
+//   k_adam    sums the partials (in FP64), applies Adam to the FP32 master parameters and
+//             refreshes the bf16 operand copies of each weight
 // The loss is the mean over samples and the 8 outputs of (y - (t - mu_out) / sig_out)^2.
 #include <hip/hip_runtime.h>
 
@@ -280,8 +281,7 @@ __device__ __forceinline__ void repack(MlpPacked *net, int i, float p) {
   }
 }
 
-// blockDim.x / 64 threads per parameter (adam_parts), which share its partials (summed in
-// FP64)
+// blockDim.x / 64 threads per parameter (adam_parts), which share its partials
 __global__ void __launch_bounds__(64 * kAdamParts)
 k_adam(const float *__restrict__ partials, int nparts, float *P, float *m, float *v,
        float *grad_out, MlpPacked *net, int step, float lr, float beta1, float beta2, float eps) {
