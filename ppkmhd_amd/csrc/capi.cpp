@@ -299,16 +299,16 @@ int launch_step(ppk_mhd_t *h, double dt, int dt_mode, int check_finished) {
     h->nparts = ppk::fused_cfl_parts(p);
   }
   if (later) HIP_CHECK(h, K.set_dt(h->ctrl, h->parts, h->nparts, dt, mode, h->p.cfl, s));
+  h->cfl_valid = cfl && (!march || ppk::march_folds_cfl(p));
   if (march) {
     HIP_CHECK(h, (p.dim == 3 ? K.march_godunov : K.march2d_godunov)(
-                     p, in, out, h->parts, h->ctrl, h->mirror, cfl ? 1 : 0, s, tm));
-    if (cfl) h->nparts = (int)ppk::march_blocks(p);
+                     p, in, out, h->parts, h->ctrl, h->mirror, h->cfl_valid ? 1 : 0, s, tm));
+    if (h->cfl_valid) h->nparts = (int)ppk::march_blocks(p);
   } else {
     HIP_CHECK(h, K.fused_godunov(p, in, out, h->fw, h->parts, h->ctrl, h->mirror, cfl ? 1 : 0, s,
                                  tm));
     if (cfl) h->nparts = ppk::fused_cfl_parts(p);
   }
-  h->cfl_valid = cfl;
   return PPK_OK;
 }
 

@@ -235,7 +235,8 @@ __device__ __forceinline__ double march2d_wave(const double *__restrict__ Uin,
           for (int v = 0; v < 8; ++v) Uout[c + v * vs] = u[v];
           if (fold) {
             // new face fields of the +1 neighbours; past the last cell the next ghost fill's
-            // (a periodic ghost column / row has its image's records, hence its CT value)
+            // (where both faces of a direction are periodic, a ghost column / row has its image's
+            // records, hence its CT value; other periodic upper faces: march_folds_cfl)
             double mx = ax, my = bn;
             if (i + 1 == p.isize - p.gw && p.bc[1] != PPK_BC_PERIODIC)
               mx = p.bc[1] == PPK_BC_DIRICHLET ? -u[IA] : u[IA];

@@ -553,6 +553,7 @@ struct MarchThread {
   // CFL term of the new cell of plane r-1 (after the new A / B of the neighbours are in LDS):
   // its primitive needs the new face fields of its +1 neighbours, or past the last interior
   // cell the values the next ghost fill puts there (fusedk::update_cell)
+  // (upper periodic faces: only where the lower one is periodic too, march_folds_cfl)
   PPK_HD double cfl_term(const DevParams &p, const double *lds, int sa, int r) {
     if (!ocol) return 0.0;
     const double *sC = lds + sa * kSlot + kSlotE;
