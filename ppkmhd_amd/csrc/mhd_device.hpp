@@ -11,6 +11,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <limits>
 
 #include "ppkmhd_amd.h"
 
@@ -68,9 +69,10 @@ PPK_HD bool sign_bit(R x) { return __builtin_signbit(x); }
 //    MI355X, over log-uniform inputs in [2^-40, 2^40] (ppk_mhd_math_selfcheck), the refined
 //    reciprocal and square root equal the IEEE results and the inverse square root is within
 //    1 ulp; each costs 4-8 instructions where the IEEE sequences with range scaling take
-//    11-14.  Inputs here are positive normal numbers (densities, pressures,
-//    wave-speed differences); sqrt(0) is 0, other zero and non-finite inputs are not
-//    handled like IEEE.
+//    11-14.  Inputs must be normal numbers (densities, pressures, wave-speed differences;
+//    whoever feeds a product that can underflow, as the EMF's Alfven speeds, keeps it normal);
+//    the inverse root is within 1 ulp over all positive ones.  sqrt(0) is 0, other zero,
+//    subnormal and non-finite inputs are not handled like IEEE.
 #ifdef PPK_EXACT_DIV
 constexpr bool kSharedRecip = false;
 #else
@@ -658,11 +660,16 @@ PPK_HD R mag_riemann2d_hlld(const St<R> &qLL, const St<R> &qRL,
     // The larger of |A| / sqrt(rho*_x) and |A*| / sqrt(rho*), with rho*_x = rho fx, A* = A fy and
     // rho* = rho fx fy, is the root of A^2 max(1, fy) / (rho fx); of two states the larger
     // fraction is found by cross multiplication, and sqrt(n / d) = n rsq(n d): one inverse
-    // square root per side instead of four.  n = 0 gives a NaN, which the maximum drops.
+    // square root per side instead of four.  A vanishing field makes n d subnormal or 0, which the
+    // inverse root must not see (n > 0 times an infinity): the smallest normal number added to
+    // it (in the same FMA; nothing changes above 2^54 times that) makes the speed about 0 there,
+    // so that the maximum is smallc.  Squared fields that underflow, |B| below 1e-154 (float:
+    // 1e-19), count as 0.  d < 0, a star density that is not physical, gives a NaN as its
+    // square root did, and the maximum drops it.
     const auto alfven = [&](R n1, R d1, R n2, R d2) {
       const bool first = n1 * d2 > n2 * d1;
       const R n = first ? n1 : n2, d = first ? d1 : d2;
-      return dmax(over_sqrt(n, n * d), smallc);
+      return dmax(over_sqrt(n, n * d + std::numeric_limits<R>::min()), smallc);
     };
     const R one = R(1);
     const R fxLL = (SL - uLL) * iSLu, fxLR = (SL - uLR) * iSLu;

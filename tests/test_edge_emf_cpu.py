@@ -1,0 +1,42 @@
+"""The default build's solver forms against the reference's expressions (both from mhd_device.hpp,
+built for the host) where a field component vanishes: 0, or so small that its square is subnormal
+or 0.  Such components occur ahead of a front in a component that starts at 0."""
+import os
+import subprocess
+
+import numpy as np
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+SRC = os.path.join(ROOT, "tests", "cxx", "edge_emf.cpp")
+
+
+@pytest.fixture(scope="module")
+def run(tmp_path_factory):
+    d = tmp_path_factory.mktemp("edge")
+    out = {}
+    for name, flags in (("lean", []), ("ref", ["-DPPK_KEEP_ROUNDING"])):
+        exe = str(d / name)
+        cmd = ["/opt/rocm/bin/hipcc", "--offload-host-only", "-std=c++17", "-O1", *flags,
+               "-ffp-contract=off", "-I", os.path.join(ROOT, "include"),
+               "-I", os.path.join(ROOT, "ppkmhd_amd", "csrc"), SRC, "-o", exe]
+        r = subprocess.run(cmd, capture_output=True, text=True)
+        assert r.returncode == 0, r.stderr[-4000:]
+        out[name] = exe
+
+    def both(*args):
+        res = []
+        for name in ("lean", "ref"):
+            r = subprocess.run([out[name], *map(str, args)], capture_output=True, text=True)
+            assert r.returncode == 0, r.stderr[-4000:]
+            res.append(np.array([l.split() for l in r.stdout.splitlines()], dtype=np.float64))
+        return res
+    return both
+
+
+def test_vanishing_fields(run):
+    lean, ref = run("vanishing", 20000)
+    assert np.isfinite(ref).all() and np.isfinite(lean).all()
+    # EMFs are u B of values up to 1; the forms differ by roundings of some tens of operations
+    for col, eps in ((0, 2.0 ** -53), (1, 2.0 ** -24)):
+        assert np.abs(lean[:, col] - ref[:, col]).max() < 200 * eps

@@ -44,3 +44,17 @@ def test_reciprocal_and_sqrt_equal_ieee(gpu):
 def test_sqrt_of_zero(gpu):
     _, sqrt, _ = selfcheck(gpu, np.array([0.0, 4.0]))
     assert sqrt[0] == 0.0 and sqrt[1] == 2.0
+
+
+def test_inverse_root_of_every_normal_number(gpu):
+    """1/sqrt(x) within one unit in the last place from the smallest normal number (which the
+    EMF's Alfven speeds clamp to) to the largest."""
+    rng = np.random.default_rng(1)
+    p2 = np.exp2(np.arange(-1022, 1024, dtype=np.float64))
+    x = np.concatenate([np.exp2(rng.uniform(-1022.0, 1024.0, 1_000_000)), p2,
+                        np.nextafter(p2[1:], 0.0), np.nextafter(p2, np.inf),
+                        [np.finfo(np.float64).max]])
+    _, _, rsq = selfcheck(gpu, np.ascontiguousarray(x))
+    ref = (1.0 / np.sqrt(x.astype(np.longdouble))).astype(np.float64)
+    ulps = np.abs(rsq - ref) / np.spacing(ref)
+    assert ulps.max() <= 1.0, f"off by {ulps.max()} ulp at {x[ulps.argmax()]}"
