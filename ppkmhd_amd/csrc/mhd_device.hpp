@@ -182,20 +182,6 @@ PPK_HD R max5(R a0, R a1, R a2, R a3, R a4) {
   return r;
 }
 
-// 1/a and 1/b from one reciprocal (neither may be zero or infinite): a product's rounding more
-// than two reciprocals, 10 instead of 14 issue slots on the GPU
-template <class R>
-PPK_HD void recip2(R a, R b, R &ia, R &ib) {
-  if (kLean) {
-    const R i = recip(a * b);
-    ia = b * i;
-    ib = a * i;
-  } else {
-    ia = recip(a);
-    ib = recip(b);
-  }
-}
-
 // square of the fast magnetosonic speed along dir, reference src/shared/mhd_utils.h:89-117
 template <class R>
 PPK_HD R speed_fast_sq(const St<R> &q, int dir, R gamma0) {
@@ -362,8 +348,7 @@ PPK_HD void riemann_hlld(St<R> &qleft, St<R> &qright, St<R> &flux,
     return a * a > R(0) && (kSharedRecip ? dabs(estar - a * a) <= R(1e-8) * (a * a)
                                          : dabs(estar / (a * a) - R(1)) <= R(1e-8));
   };
-  R isl, isr;
-  recip2(sl - ustar, sr - ustar, isl, isr);
+  const R isl = recip(sl - ustar), isr = recip(sr - ustar);
   R rstarl = divr(rl * (sl - ul), sl - ustar, isl);
   R estar = rl * (sl - ul) * (sl - ustar) - a * a;
   R el = rl * (sl - ul) * (sl - ul) - a * a;
@@ -597,18 +582,15 @@ PPK_HD R mag_riemann2d_hlld(const St<R> &qLL, const St<R> &qRL,
   R rcRRy = rRR * (ST - vRR);
 
   const R rcx = rcLLx + rcLRx + rcRLx + rcRRx, rcy = rcLLy + rcLRy + rcRLy + rcRRy;
-  R ircx, ircy;
-  recip2(rcx, rcy, ircx, ircy);
   R ustar = divr(rcLLx * uLL + rcLRx * uLR + rcRLx * uRL + rcRRx * uRR +
                      (PtotLL - PtotRL + PtotLR - PtotRR),
-                 rcx, ircx);
+                 rcx, recip(rcx));
   R vstar = divr(rcLLy * vLL + rcLRy * vLR + rcRLy * vRL + rcRRy * vRR +
                      (PtotLL - PtotLR + PtotRL - PtotRR),
-                 rcy, ircy);
+                 rcy, recip(rcy));
 
-  R iSLu, iSRu, iSBv, iSTv;
-  recip2(SL - ustar, SR - ustar, iSLu, iSRu);
-  recip2(SB - vstar, ST - vstar, iSBv, iSTv);
+  const R iSLu = recip(SL - ustar), iSRu = recip(SR - ustar);
+  const R iSBv = recip(SB - vstar), iSTv = recip(ST - vstar);
 
   R rstarLLx = divr(rLL * (SL - uLL), SL - ustar, iSLu);
   R BstarLL = kLean ? bLL * ((SL - uLL) * iSLu)
@@ -699,8 +681,7 @@ PPK_HD R mag_riemann2d_hlld(const St<R> &qLL, const St<R> &qRL,
   R SAB = dmin(vstar - calfvenB, R(0));
   R SAT = dmax(vstar + calfvenT, R(0));
 
-  R iSAx, iSAy;
-  recip2(SAR - SAL, SAT - SAB, iSAx, iSAy);
+  const R iSAx = recip(SAR - SAL), iSAy = recip(SAT - SAB);
   R AstarT = divr(SAR * AstarRR - SAL * AstarLR, SAR - SAL, iSAx);
   R AstarB = divr(SAR * AstarRL - SAL * AstarLL, SAR - SAL, iSAx);
   R BstarR = divr(SAT * BstarRR - SAB * BstarRL, SAT - SAB, iSAy);

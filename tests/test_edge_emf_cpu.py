@@ -1,6 +1,7 @@
 """The default build's solver forms against the reference's expressions (both from mhd_device.hpp,
 built for the host) where a field component vanishes: 0, or so small that its square is subnormal
-or 0.  Such components occur ahead of a front in a component that starts at 0."""
+or 0, as ahead of a front in a component that starts at 0; and where wave speeds coincide because
+the sound speed is lost in the velocity, so that a denominator of one side or direction is 0."""
 import os
 import subprocess
 
@@ -40,3 +41,14 @@ def test_vanishing_fields(run):
     # EMFs are u B of values up to 1; the forms differ by roundings of some tens of operations
     for col, eps in ((0, 2.0 ** -53), (1, 2.0 ** -24)):
         assert np.abs(lean[:, col] - ref[:, col]).max() < 200 * eps
+
+
+@pytest.mark.parametrize("mode", ["cold", "stream"])
+def test_coinciding_waves(run, mode):
+    """A side or direction whose denominator is 0 leaves the others as they are: what is finite with
+    the reference's expressions is finite, and equal to the roundings of some tens of operations."""
+    lean, ref = run(mode, 2000)
+    ok = np.isfinite(ref)
+    assert ok.any() and np.isfinite(lean[ok]).all()
+    scale = np.abs(np.where(ok, ref, 0.0)).max(0)
+    assert (np.abs(lean - ref)[ok] <= (200 * 2.0 ** -53 * scale * np.ones_like(ref))[ok]).all()
