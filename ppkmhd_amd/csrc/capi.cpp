@@ -67,20 +67,6 @@ bool fused_supported(const DevParams &p, int precision, int kernel_path) {
   return precision == PPK_FP64 || precision == PPK_FP64_STRICT || precision == PPK_FP32_BULK;
 }
 
-void march2d_shape(DevParams &p, int cus) {
-  double best = 0.0;
-  for (int lw = 64; lw >= 32; lw /= 2)
-    for (int rows = 1; rows <= p.ny; ++rows) {
-      const double t = march2d_time((double)march2d_waves(p, lw, rows), rows, cus);
-      if (best == 0.0 || t < best * 0.999) {
-        best = t;
-        p.march_lw = lw;
-        p.march_rows = rows;
-      }
-    }
-  p.march = (int)march2d_waves(p, p.march_lw, p.march_rows);
-}
-
 }  // namespace ppk
 
 struct ppk_mhd_solver {

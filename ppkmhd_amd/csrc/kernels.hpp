@@ -210,7 +210,20 @@ inline double march2d_time(double waves, int rows, int cus) {
   const double per = waves <= simds ? 1.0 : (double)(long long)((waves + simds - 1.0) / simds);
   return per <= 1.0 ? rows + 3.1 : 0.93 * per * (rows + 1.6);
 }
-void march2d_shape(DevParams &p, int cus);  // sets march_lw, march_rows and march
+// sets march_lw, march_rows and march
+inline void march2d_shape(DevParams &p, int cus) {
+  double best = 0.0;
+  for (int lw = 64; lw >= 32; lw /= 2)
+    for (int rows = 1; rows <= p.ny; ++rows) {
+      const double t = march2d_time((double)march2d_waves(p, lw, rows), rows, cus);
+      if (best == 0.0 || t < best * 0.999) {
+        best = t;
+        p.march_lw = lw;
+        p.march_rows = rows;
+      }
+    }
+  p.march = (int)march2d_waves(p, p.march_lw, p.march_rows);
+}
 // Whether the single-pass steps can give the CFL maxima of the state they write.  Behind the last
 // cell of a direction they take the new face field of the ghost cell as computed from that last
 // cell.  With both faces periodic this is what the next ghost fill puts there; with only the upper

@@ -33,7 +33,8 @@ def pair(kind, path, tEnd):
 
 
 @pytest.mark.parametrize("kind", ["mhd2", "mhd3", "hydro"])
-@pytest.mark.parametrize("path", [A.PATH_AUTO, A.PATH_FUSED_RECORDS, A.PATH_STAGED])
+@pytest.mark.parametrize("path", [A.PATH_AUTO, A.PATH_FUSED, A.PATH_FUSED_RECORDS,
+                                  A.PATH_STAGED])
 def test_time_follows_every_call(oracle, gpu, kind, path):
     o, g = pair(kind, path, 1.0)
     with g:
@@ -74,7 +75,7 @@ def test_more_partials_than_the_prologue_reduces(gpu):
     p = make_params(3, 128, 128, 128, gamma0=5 / 3, cfl=0.8, tEnd=1.0, precision=A.FP64_STRICT)
     pr = default_problem(A.PROBLEM_BLAST, p)
     out = []
-    for path in (A.PATH_AUTO, A.PATH_FUSED_RECORDS):
+    for path in (A.PATH_FUSED, A.PATH_FUSED_RECORDS):
         p.kernel_path = path
         with SolverMHDMuscl(p, pr) as s:
             s.run(4)

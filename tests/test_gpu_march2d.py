@@ -1,7 +1,8 @@
 """The single-pass 2D step where its strips end: widths around multiples of the 60 and 28 output
-columns, heights of one strip, ragged last strips, every boundary type.  The strict build is
-bit-identical to the oracle (ghosts, t and dt included) and, where strips hold many rows, to the
-three-kernel form."""
+columns of a strip, on grids whose strips are 64 columns of one row (SMALL) and on grids with strips
+of 32 columns, of several rows, with a ragged last strip (LONG; test_march2d_shape_cpu.py holds the
+shapes), with every boundary type and solver.  The strict build is bit-identical to the oracle
+(ghosts, t and dt included) and, where strips hold many rows, to the three-kernel form."""
 import numpy as np
 import pytest
 
@@ -19,6 +20,11 @@ def case(nx, ny, bc, **kw):
     return p, default_problem(A.PROBLEM_ORSZAG_TANG, p)
 
 
+SMALL = [(3, 3), (28, 5), (29, 7), (57, 4), (60, 3), (61, 16), (120, 9), (121, 33), (5, 131)]
+LONG = [(3, 1273), (67, 1272), (3, 5003), (61, 2001), (61, 2503), (85, 1272), (29, 2503),
+        (121, 1272), (29, 5003)]
+
+
 def solver(p, pr, path):
     from ppkmhd_amd.solver import SolverMHDMuscl
     q = A.Params.from_buffer_copy(p)
@@ -26,18 +32,18 @@ def solver(p, pr, path):
     return SolverMHDMuscl(q, pr)
 
 
-@pytest.mark.parametrize("nx,ny", [(3, 3), (28, 5), (29, 7), (57, 4), (60, 3), (61, 16),
-                                   (120, 9), (121, 33), (5, 131)])
+@pytest.mark.parametrize("nx,ny", SMALL + LONG)
 @pytest.mark.parametrize("bc,kw", [
     (P, {}),
     ([P, P, N, N, P, P], dict(slope_type=2.0, riemann=A.RIEMANN_HLL)),
     ([N, N, D, N, P, P], dict(riemann=A.RIEMANN_LLF)),
+    ([D, N, N, D, P, P], dict(slope_type=2.0)),
 ])
 def test_strict_equals_oracle(oracle, gpu, nx, ny, bc, kw):
     p, pr = case(nx, ny, bc, **kw)
     o = oracle.Solver(p)
     o.init_problem(pr)
-    with solver(p, pr, A.PATH_AUTO) as g:
+    with solver(p, pr, A.PATH_FUSED) as g:
         for _ in range(4):
             o.step(0.0, A.DT_CFL)
             g.step(0.0, A.DT_CFL)
@@ -48,7 +54,7 @@ def test_strict_equals_oracle(oracle, gpu, nx, ny, bc, kw):
 @pytest.mark.parametrize("nx,ny", [(640, 480), (1021, 517), (1500, 1301)])
 def test_strict_equals_three_kernel_form(gpu, nx, ny):
     p, pr = case(nx, ny, [P, P, N, N, P, P], slope_type=2.0)
-    with solver(p, pr, A.PATH_AUTO) as a, solver(p, pr, A.PATH_FUSED_RECORDS) as b:
+    with solver(p, pr, A.PATH_FUSED) as a, solver(p, pr, A.PATH_FUSED_RECORDS) as b:
         for s in (a, b):
             s.run(3)
             s.step(1e-5, A.DT_FIXED)

@@ -15,9 +15,9 @@ from test_golden_cpu import load_case
 
 pytestmark = pytest.mark.gpu
 
-# staged; the default (3D FP64: the single-pass kernel; 2D: the three-kernel fused form); the
-# three-kernel fused form (half-step records in HBM) in 3D too
-PATHS = [A.PATH_STAGED, A.PATH_AUTO, A.PATH_FUSED_RECORDS]
+# staged; the default (the faster of the two fused forms by size: the three-kernel form on small 3D
+# grids); the single-pass kernels; the three-kernel form (half-step records in HBM)
+PATHS = [A.PATH_STAGED, A.PATH_AUTO, A.PATH_FUSED, A.PATH_FUSED_RECORDS]
 
 
 def solver(p, pr=None):
@@ -216,7 +216,7 @@ def test_fast_1000_steps_l1(oracle, gpu, path):
     assert abs(g.m_t - o.time()[0]) <= 1e-12 * o.time()[0]
 
 
-@pytest.mark.parametrize("path", [A.PATH_AUTO, A.PATH_FUSED_RECORDS])
+@pytest.mark.parametrize("path", [A.PATH_AUTO, A.PATH_FUSED, A.PATH_FUSED_RECORDS])
 def test_fast_1000_steps_l1_3d(oracle, gpu, path):
     """3D blast 24^3, 1000 CFL steps (the single-pass kernel and the three-kernel form):
     relative L1 <= 1e-10 against the oracle, div B at roundoff."""
@@ -316,10 +316,12 @@ def test_compute_dt_matches_oracle(oracle, gpu):
 
 @pytest.mark.parametrize("case", ["ot2d", "blast3d"])
 @pytest.mark.parametrize("precision", [A.FP64, A.FP64_STRICT])
-def test_restart_continues_bit_identically(gpu, tmp_path, case, precision):
+@pytest.mark.parametrize("path", [A.PATH_AUTO, A.PATH_FUSED])
+def test_restart_continues_bit_identically(gpu, tmp_path, case, precision, path):
     """Stop after 4 CFL steps, save, load into a fresh solver and run 6 more: the state, t, dt
     and iteration equal those of 10 uninterrupted steps, bit for bit."""
-    p, pr = ot2d(40, 36, precision=precision) if case == "ot2d" else blast3d(14, precision=precision)
+    kw = dict(precision=precision, kernel_path=path)
+    p, pr = ot2d(40, 36, **kw) if case == "ot2d" else blast3d(14, **kw)
     a = solver(p, pr)
     a.run(10)
     b = solver(p, pr)
