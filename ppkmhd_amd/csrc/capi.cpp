@@ -381,11 +381,13 @@ int ppk_mhd_create(const ppk_mhd_params *params, ppk_mhd_t **handle) {
   if (h->fused && params->precision != PPK_FP32_BULK &&
       params->kernel_path != PPK_PATH_FUSED_RECORDS) {
     if (params->dim == 3)
-      h->dp.march = params->kernel_path == PPK_PATH_FUSED || ppk::march_pays(h->dp, cus)
-                        ? ppk::march_nblk(h->dp, cus)
-                        : 0;
+      h->dp.march = ppk::march_nblk(h->dp, cus);
     else
       ppk::march2d_shape(h->dp, cus);
+    const bool pays = params->dim == 3 ? ppk::march_pays(h->dp, cus)
+                                       : ppk::march2d_pays(h->dp, cus, params->precision ==
+                                                                           PPK_FP64_STRICT);
+    if (params->kernel_path != PPK_PATH_FUSED && !pays) h->dp.march = 0;
   }
   if (params->kernel_path == PPK_PATH_FUSED && !h->fused) {
     delete h;

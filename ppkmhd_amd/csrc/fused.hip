@@ -1,6 +1,7 @@
 // Fused form of the MHD step: three stages per time step in place of the reference's seven.
 // The FP32-bulk form, the surrogate and the batch run it; plain FP64 steps run the single-pass
-// kernels (march3d.hip, march2d.hip) except in small 3D boxes (march_pays).
+// kernels (march3d.hip, march2d.hip) except where this form is the faster one (march_pays,
+// march2d_pays).
 //
 //   k_half3d / k_half2d        LDS-tiled: primitives, edge electric field, transverse
 //                              face-field slopes and the Hancock half step of a tile of cells;

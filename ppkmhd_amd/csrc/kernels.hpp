@@ -224,6 +224,25 @@ inline void march2d_shape(DevParams &p, int cus) {
     }
   p.march = (int)march2d_waves(p, p.march_lw, p.march_rows);
 }
+// PPK_PATH_AUTO: whether the single-pass 2D step is the faster form (shape set by march2d_shape).
+// Times of a step in us: the single pass by the rows of a strip and the waves per SIMD, the
+// three-kernel form by the padded cells, dearer per cell once its records leave the caches.
+// Measured single-pass / three-kernel, default build: 64^2 19 / 24, 256^2 27 / 31, 2048^2 299 / 880,
+// 16x4096 31 / 34, 5x20000 65 / 57, 5x200000 438 / 577; strict build: 64^2 30 / 29, 256^2 48 / 40,
+// 400^2 55 / 59, 2048^2 665 / 1008, 16x4096 52 / 42, 67x1272 52 / 41, 5x20000 129 / 72, 30x30000
+// 303 / 280.  Strips of a narrow grid leave most lanes idle; the strict build's exact quotients
+// cost the single pass, bound by issue at few waves, more than the other form.
+inline bool march2d_pays(const DevParams &p, int cus, bool strict) {
+  const double simds = 4.0 * (cus > 0 ? cus : 256);
+  const double per = p.march <= simds ? 1.0 : (double)(long long)((p.march + simds - 1.0) / simds);
+  const double rows = p.march_rows * (p.march_lw == 32 ? 1.12 : 1.0);
+  const double k = (double)p.isize * p.jsize * 1e-3, far = k > 700.0 ? k - 700.0 : 0.0;
+  if (strict)
+    return (per <= 1.0 ? 18.5 + 11.3 * rows : 34.0 + 8.75 * per * rows) <
+           25.0 + 0.2 * k + 0.045 * far;
+  return (per <= 1.0 ? 14.5 + 5.0 * rows : 22.0 + 3.9 * per * rows) <
+         22.0 + 0.14 * k + 0.1 * far;
+}
 // Whether the single-pass steps can give the CFL maxima of the state they write.  Behind the last
 // cell of a direction they take the new face field of the ghost cell as computed from that last
 // cell.  With both faces periodic this is what the next ghost fill puts there; with only the upper

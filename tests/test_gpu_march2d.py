@@ -61,3 +61,16 @@ def test_strict_equals_three_kernel_form(gpu, nx, ny):
             s.run(2)
         assert np.array_equal(a.download(), b.download())
         assert a.time() == b.time()
+
+
+@pytest.mark.parametrize("nx,ny", [(64, 64), (16, 4096), (5, 20000), (400, 400)])
+def test_auto_gives_the_bits_of_either_form(gpu, nx, ny):
+    """AUTO takes the faster form by size (march2d_pays): here both forms occur."""
+    p, pr = case(nx, ny, [N, N, P, P, P, P])
+    out = []
+    for path in (A.PATH_AUTO, A.PATH_FUSED, A.PATH_FUSED_RECORDS):
+        with solver(p, pr, path) as s:
+            s.run(4)
+            out.append((s.time(), s.download()))
+    for t, U in out[1:]:
+        assert t == out[0][0] and np.array_equal(U, out[0][1])
