@@ -215,6 +215,7 @@ inline void march2d_shape(DevParams &p, int cus) {
   double best = 0.0;
   for (int lw = 64; lw >= 32; lw /= 2)
     for (int rows = 1; rows <= p.ny; ++rows) {
+      if (best > 0.0 && rows + 2.9 > best) break;  // no launch takes less than its rows + 2.9
       const double t = march2d_time((double)march2d_waves(p, lw, rows), rows, cus);
       if (best == 0.0 || t < best * 0.999) {
         best = t;
