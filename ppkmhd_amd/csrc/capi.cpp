@@ -262,7 +262,7 @@ int launch_step(ppk_mhd_t *h, double dt, int dt_mode, int check_finished) {
   const int mode = cfl ? ppk::SETDT_CFL : ppk::SETDT_FIXED;
   if (!h->fused) {
     HIP_CHECK(h, K.begin(h->ctrl, check_finished, s));
-    HIP_CHECK(h, K.boundaries(p, in, nullptr, h->ctrl, s, tm));
+    HIP_CHECK(h, K.boundaries(p, in, h->ctrl, s, tm));
     const int nparts = ppk::cfl_blocks(p);
     HIP_CHECK(h, K.prim_dt(p, in, h->Q, h->parts, h->ctrl, cfl ? 1 : 0, s, tm));
     HIP_CHECK(h, K.set_dt(h->ctrl, h->parts, nparts, dt, mode, h->p.cfl, s));
@@ -559,7 +559,7 @@ int ppk_mhd_stream(ppk_mhd_t *h, void **stream) {
 int ppk_mhd_make_boundaries(ppk_mhd_t *h) {
   if (!h) return fail(h, PPK_ERR_INVALID_ARGUMENT, "NULL handle");
   HIP_CHECK(h, h->K->begin(h->ctrl, 0, h->stream));
-  HIP_CHECK(h, h->K->boundaries(h->dp, h->cur(), nullptr, h->ctrl, h->stream, h->tm()));
+  HIP_CHECK(h, h->K->boundaries(h->dp, h->cur(), h->ctrl, h->stream, h->tm()));
   return PPK_OK;
 }
 
@@ -567,7 +567,7 @@ int ppk_mhd_compute_dt(ppk_mhd_t *h, double *dt) {
   if (!h || !dt) return fail(h, PPK_ERR_INVALID_ARGUMENT, "NULL argument");
   // the dt the next step would take: ghost fill, primitives, CFL max (no tEnd clamp)
   HIP_CHECK(h, h->K->begin(h->ctrl, 0, h->stream));
-  HIP_CHECK(h, h->K->boundaries(h->dp, h->cur(), nullptr, h->ctrl, h->stream, h->tm()));
+  HIP_CHECK(h, h->K->boundaries(h->dp, h->cur(), h->ctrl, h->stream, h->tm()));
   if (h->fused) {
     HIP_CHECK(h, h->K->fused_cfl(h->dp, h->cur(), h->parts, h->ctrl, h->stream, h->tm()));
     h->cfl_valid = true;
@@ -602,7 +602,7 @@ int ppk_mhd_dump_faces(ppk_mhd_t *h, ppk_faceset_t *set, int stride, int phase,
   if (!alloc_records(h)) return fail(h, PPK_ERR_OUT_OF_MEMORY, "device allocation failed");
   // the faces the next CFL step will solve: ghost fill, CFL dt, half-step records
   HIP_CHECK(h, h->K->begin(h->ctrl, 1, h->stream));
-  HIP_CHECK(h, h->K->boundaries(h->dp, h->cur(), nullptr, h->ctrl, h->stream, h->tm()));
+  HIP_CHECK(h, h->K->boundaries(h->dp, h->cur(), h->ctrl, h->stream, h->tm()));
   HIP_CHECK(h, h->K->fused_cfl(h->dp, h->cur(), h->parts, h->ctrl, h->stream, h->tm()));
   HIP_CHECK(h, h->K->set_dt(h->ctrl, h->parts, ppk::fused_cfl_parts(h->dp), 0.0,
                             ppk::SETDT_CFL, h->p.cfl, h->stream));

@@ -153,13 +153,13 @@ __device__ __forceinline__ double inv_dt_cell(const HSt<NV> &u, const G3 &g, con
 // Neumann copies the first interior cell, periodic wraps.  One launch where three direction
 // passes took 37 us (256 x 192 x 128).
 template <int NV>
-__global__ void __launch_bounds__(kBlock) k_hbnd(double *__restrict__ U, double *__restrict__ C,
-                                                 HydroDev h, const double *ctrl) {
+__global__ void __launch_bounds__(kBlock) k_hbnd(double *__restrict__ U, HydroDev h,
+                                                 const double *ctrl) {
   if (!active(ctrl)) return;
   const long long total = ghost_shell_cells(h);
   for (long long t = blockIdx.x * (long long)blockDim.x + threadIdx.x; t < total;
        t += (long long)gridDim.x * blockDim.x)
-    ghost_shell_element<NV>(U, h, t, C);
+    ghost_shell_element<NV>(U, h, t, nullptr);
 }
 template <int NV>
 __global__ void __launch_bounds__(kBlock) k_hprologue(double *__restrict__ U,
@@ -632,13 +632,12 @@ int fused3d_blocks(const HydroDev &h) {
 // -------------------------------------------------------------------------------------------
 // launchers
 // -------------------------------------------------------------------------------------------
-hipError_t hydro_boundaries(const HydroDev &h, double *U, double *copy, const double *ctrl,
-                            hipStream_t s) {
+hipError_t hydro_boundaries(const HydroDev &h, double *U, const double *ctrl, hipStream_t s) {
   const dim3 g(grid_for(ghost_shell_cells(h))), b(kBlock);
   if (h.dim == 3)
-    hipLaunchKernelGGL(k_hbnd<5>, g, b, 0, s, U, copy, h, ctrl);
+    hipLaunchKernelGGL(k_hbnd<5>, g, b, 0, s, U, h, ctrl);
   else
-    hipLaunchKernelGGL(k_hbnd<4>, g, b, 0, s, U, copy, h, ctrl);
+    hipLaunchKernelGGL(k_hbnd<4>, g, b, 0, s, U, h, ctrl);
   return hipGetLastError();
 }
 

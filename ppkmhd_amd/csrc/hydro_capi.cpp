@@ -596,7 +596,7 @@ int hlaunch_step(ppk_hydro_t *h, double dt, int dt_mode, int check_finished) {
     h->cfl_valid = cfl;
   } else {
     HHIP(h, K.begin(h->ctrl, check_finished, s));
-    PPK_TIMED(tm, ppk::HS_BOUNDARIES, HHIP(h, H.boundaries(d, in, nullptr, h->ctrl, s)));
+    PPK_TIMED(tm, ppk::HS_BOUNDARIES, HHIP(h, H.boundaries(d, in, h->ctrl, s)));
     PPK_TIMED(tm, ppk::HS_PRIM_DT,
               HHIP(h, H.prim_dt(d, in, h->Q, h->parts, h->ctrl, cfl ? 1 : 0, s)));
     PPK_TIMED(tm, ppk::HS_CONTROL,
@@ -802,7 +802,7 @@ int ppk_hydro_device_state(ppk_hydro_t *h, double **dU) {
 int ppk_hydro_make_boundaries(ppk_hydro_t *h) {
   if (!h) return hfail(h, PPK_ERR_INVALID_ARGUMENT, "NULL handle");
   HHIP(h, h->K->begin(h->ctrl, 0, h->stream));
-  HHIP(h, h->H->boundaries(h->hd, h->cur(), nullptr, h->ctrl, h->stream));
+  HHIP(h, h->H->boundaries(h->hd, h->cur(), h->ctrl, h->stream));
   return PPK_OK;
 }
 

@@ -43,11 +43,11 @@ constexpr int kHydroRows3 = kHydroBlockRows3 - 2;
 
 #define PPK_DECLARE_HYDRO(NS)                                                                    \
   namespace NS {                                                                                 \
-  /* ghost fill of U in one pass (the values of x, then y, then z passes); with copy != nullptr every ghost value is also        \
-     written there (the next state's ghosts = this state's, as the reference's deep copy) */    \
-  hipError_t hydro_boundaries(const HydroDev &h, double *U, double *copy, const double *ctrl,    \
-                              hipStream_t s);                                                    \
-  /* the finished test, the ghost fill and dt in one launch (staged_prologue) */                 \
+  /* ghost fill of U in one pass (the values of x, then y, then z passes) */                     \
+  hipError_t hydro_boundaries(const HydroDev &h, double *U, const double *ctrl, hipStream_t s);  \
+  /* the finished test, the ghost fill and dt in one launch (staged_prologue); with copy !=      \
+     nullptr every ghost value is also written there (the next state's ghosts = this state's,    \
+     as the reference's deep copy) */                                                            \
   hipError_t hydro_prologue(const HydroDev &h, double *U, double *copy, double *ctrl,            \
                             const double *parts, int nparts, double fixed_dt, int mode,          \
                             double cfl, int check_finished, hipStream_t s);                      \

@@ -284,11 +284,12 @@ struct BatchMember {
 
 #define PPK_DECLARE_KERNELS(NS)                                                                  \
   namespace NS {                                                                                 \
-  /* ghost fill of U; copy (may be null) receives the same ghost values */                     \
-  hipError_t staged_boundaries(const DevParams &p, double *U, double *copy, const double *ctrl,  \
+  /* ghost fill of U */                                                                          \
+  hipError_t staged_boundaries(const DevParams &p, double *U, const double *ctrl,                \
                                hipStream_t s, StageTimer *tm);                                   \
-  /* the finished test, the ghost fill (copy as above) and dt in one launch; nparts at most      \
-     kPrologueParts unless mode is SETDT_FIXED or SETDT_LATER */                                \
+  /* the finished test, the ghost fill of U and dt in one launch; copy (may be null) receives    \
+     the same ghost values; nparts at most kPrologueParts unless mode is SETDT_FIXED or          \
+     SETDT_LATER */                                                                              \
   hipError_t staged_prologue(const DevParams &p, double *U, double *copy, double *ctrl,          \
                              const double *parts, int nparts, double fixed_dt, int mode,         \
                              double cfl, int check_finished, hipStream_t s, StageTimer *tm);     \

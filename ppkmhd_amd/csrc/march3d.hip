@@ -1,7 +1,7 @@
 // Single-pass 3D MHD step: one kernel reads the state once and writes the interior of the new
 // state once (bodies and data flow: march_body.hpp).  The ghost cells of the new state are the
 // reference's deep copy of the filled input ghosts (U2 = U before the update): the step's ghost
-// fill (staged_boundaries with the new state as its copy target) writes each ghost value to
+// fill (staged_prologue with the new state as its copy target) writes each ghost value to
 // both states.
 #include <hip/hip_runtime.h>
 

@@ -46,14 +46,13 @@ __device__ __forceinline__ void decompose(const DevParams &p, long long t, int &
 // ---- ghost fill of every face, edge and corner in one pass: ghost_shell_element
 // (kernels.hpp) per ghost cell, the values of the reference's x, y, z passes
 // (src/shared/SolverBase.cpp:339-537, src/shared/BoundariesFunctors.h:534-1057) ------------
-__global__ void __launch_bounds__(kBlock) k_boundaries(double *__restrict__ U,
-                                                       double *__restrict__ copy, DevParams p,
+__global__ void __launch_bounds__(kBlock) k_boundaries(double *__restrict__ U, DevParams p,
                                                        const double *ctrl) {
   if (!active(ctrl)) return;
   const long long total = ghost_shell_cells(p);
   for (long long t = blockIdx.x * (long long)blockDim.x + threadIdx.x; t < total;
        t += (long long)gridDim.x * blockDim.x)
-    ghost_shell_element(U, p, t, copy);
+    ghost_shell_element(U, p, t, nullptr);
 }
 
 // ---- primitives over [0, size-1) per direction + CFL max over the interior ----------------
@@ -436,11 +435,11 @@ int grid_for(long long n) {
 // -------------------------------------------------------------------------------------------
 // launchers
 // -------------------------------------------------------------------------------------------
-hipError_t staged_boundaries(const DevParams &p, double *U, double *copy, const double *ctrl,
-                             hipStream_t s, StageTimer *tm) {
+hipError_t staged_boundaries(const DevParams &p, double *U, const double *ctrl, hipStream_t s,
+                             StageTimer *tm) {
   if (tm) tm->mark(ST_BOUNDARIES, true);
   hipLaunchKernelGGL(k_boundaries, dim3(grid_for(ghost_shell_cells(p))), dim3(kBlock), 0, s, U,
-                     copy, p, ctrl);
+                     p, ctrl);
   if (tm) tm->mark(ST_BOUNDARIES, false);
   return hipGetLastError();
 }
