@@ -239,16 +239,16 @@ int read_ctrl(ppk_mhd_t *h) {
   return PPK_OK;
 }
 
-// device buffers of the three-kernel fused form (records, fluxes, EMFs)
+// device buffers of the three-kernel fused form (records, fluxes, EMFs); a call after one that
+// failed allocates what is missing
 bool alloc_records(ppk_mhd_t *h) {
-  if (h->fw.rec) return true;
   const int d = h->dp.dim;
   const size_t n = (size_t)h->cells();
   const size_t es = h->dp.bulk32 ? sizeof(float) : sizeof(double);
-  return hipMalloc(&h->fw.rec, (size_t)(d == 3 ? ppk::kRec3 : ppk::kRec2) * n * es) == hipSuccess &&
-         hipMalloc(&h->fw.flux,
-                   (size_t)d * (d == 3 ? ppk::kFluxComp3 : ppk::kFluxComp2) * n * es) == hipSuccess &&
-         hipMalloc(&h->fw.emf, (size_t)(d == 3 ? 3 : 1) * n * sizeof(double)) == hipSuccess;
+  const auto need = [](auto *&p, size_t bytes) { return p || hipMalloc(&p, bytes) == hipSuccess; };
+  return need(h->fw.rec, (size_t)(d == 3 ? ppk::kRec3 : ppk::kRec2) * n * es) &&
+         need(h->fw.flux, (size_t)d * (d == 3 ? ppk::kFluxComp3 : ppk::kFluxComp2) * n * es) &&
+         need(h->fw.emf, (size_t)(d == 3 ? 3 : 1) * n * sizeof(double));
 }
 
 // one time step from cur() into nxt() (godunov_unsplit_impl), optionally gated on finished()
