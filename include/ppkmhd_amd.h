@@ -55,7 +55,7 @@ enum ppk_kernel_path {
   PPK_PATH_AUTO = 0,   /* fused kernels where available, else staged; of the fused forms the
                         * one that is faster at the grid's size                              */
   PPK_PATH_STAGED = 1, /* one kernel per reference stage, intermediates in HBM                */
-  PPK_PATH_FUSED = 2,  /* fused kernels: in FP64 the single-pass step (state read once and   
+  PPK_PATH_FUSED = 2,  /* fused kernels: in FP64 the single-pass step (state read once and
                         * written once), else the three-kernel form                          */
   PPK_PATH_FUSED_RECORDS = 3 /* the three-kernel fused form in every case (half-step records,
                         * face/edge solves, update; records and fluxes in HBM)               */
@@ -296,7 +296,9 @@ int ppk_mhd_synchronize(ppk_mhd_t *h);
  * Per-stage GPU timers, the counterpart of the reference's phase timers (TIMER_BOUNDARIES,
  * TIMER_DT, TIMER_NUM_SCHEME; src/shared/SolverBase.h:35-42, 150-157): when a stage's bit is
  * set in stage_mask, every launch of that stage is bracketed by a pair of hipEvents recorded
- * on the handle's stream.  Enabling (or disabling) clears the accumulated times.
+ * on the handle's stream.  Enabling (or disabling) clears the accumulated times.  In the fused
+ * paths the finished test, the ghost fill and dt are one launch, counted as "boundaries" (a dt
+ * launch of its own, where there are too many partial maxima for that one, is not timed).
  */
 int ppk_mhd_timers_enable(ppk_mhd_t *h, uint32_t stage_mask);
 /* Sum of the recorded durations (ms) and the number of launches of one stage (synchronizes). */
@@ -352,8 +354,12 @@ int ppk_mhd_load_state(ppk_mhd_t *h, const char *path, int64_t *time_step);
  * all members, and steps after the first replay one captured hipGraph.  Each member follows
  * its own time loop exactly as one ppk_mhd_t would with dt_mode PPK_DT_CFL (its own CFL dt,
  * clamp to tEnd, finished() test); the per-cell code is the fused path's, so its state after
- * each step equals that handle's bit for bit in PPK_FP64_STRICT (to roundoff in the other
- * precisions, where the compiler's FMA contractions may differ between the two kernels).
+ * each step equals that handle's bit for bit in PPK_FP64_STRICT.  In PPK_FP64 and PPK_FP32_BULK
+ * it equals it to roundoff: the batch runs the three-kernel form with solvers that keep the
+ * reference's expressions, the handle's take shorter ones (and FMA contractions may differ), so
+ * long chaotic runs part there; PPK_FP64_STRICT is the mode to compare entry points in.
+ * A batch pays for members too small to fill the GPU alone (in FP64, up to about 300^2 or 50^3
+ * cells); larger ones run faster one handle after another, on the single-pass kernels.
  * Replaces: a loop over the reference's driver, one SolverMHDMuscl per member
  * (src/main.cpp:130-160 with src/shared/SolverBase.cpp:161-219), for PPK_PATH_FUSED. */
 typedef struct ppk_mhd_batch ppk_mhd_batch;
@@ -492,7 +498,9 @@ int ppk_hydro_synchronize(ppk_hydro_t *h);
 int ppk_hydro_save_vtk(ppk_hydro_t *h, const char *dir, const char *prefix, int istep,
                        int ascii);
 /* Per-stage GPU timers (hipEvents on the handle's stream), as ppk_mhd_timers_*; stages:
- * 0 boundaries, 1 primitives_dt, 2 fluxes, 3 update (staged form), 4 fused, 5 control.
+ * 0 boundaries, 1 primitives_dt, 2 fluxes, 3 update (staged form), 4 fused, 5 control (dt; in the
+ * fused form only where it is a launch of its own: the first step, and grids of many partial
+ * maxima; else it is part of 0).
  * Replaces: the per-stage timers of SolverBase (src/shared/SolverBase.h:35-42, 150-157). */
 int ppk_hydro_timers_enable(ppk_hydro_t *h, uint32_t stage_mask);
 int ppk_hydro_timers_read(ppk_hydro_t *h, int stage, double *total_ms, int64_t *launches);

@@ -49,7 +49,7 @@ UNITS = [
     ("march2d.hip", "march2d_fast.o", ["-DPPK_NS=fast", "-ffp-contract=fast"]),
     ("march2d.hip", "march2d_strict.o",
      ["-DPPK_NS=strict", "-DPPK_EXACT_DIV", "-ffp-contract=off"]),
-    # ensembles keep their rounding (kLean in mhd_device.hpp)
+    # ensembles keep the rounding of earlier builds (kLean in mhd_device.hpp)
     ("batch.hip", "batch_fast.o",
      ["-DPPK_NS=fast", "-DPPK_KEEP_ROUNDING", "-ffp-contract=fast"]),
     ("batch.hip", "batch_strict.o", ["-DPPK_NS=strict", "-DPPK_EXACT_DIV", "-ffp-contract=off"]),

@@ -229,8 +229,8 @@ void batch_block_counts(const DevParams &p, int tile, long long counts[BS_COUNT]
 }
 
 // one step of every member: prologue (finished test, ghost fill, dt), on request a standalone
-// CFL pass and dt from it, the three fused stages (the last one ends the step).  Stream-ordered, no host synchronization, no memset: safe
-// to capture in a graph and replay.
+// CFL pass and dt from it, the three fused stages (the last one ends the step).  Stream-ordered,
+// no host synchronization, no memset: safe to capture in a graph and replay.
 template <class R>
 void launch_bhalf(const BatchMember *members, int nm, int dim, int tile, long long blocks,
                   hipStream_t s) {

@@ -179,6 +179,7 @@ inline int march_nblk(const DevParams &p, int cus) {
 // cut tiles); the three-kernel form takes 0.43 us per 1000 cells once its launches are paid.
 // Measured us per step, single-pass / three-kernel: 16^3 41 / 32, 32^3 45 / 42, 37x29x45 76 / 45,
 // 48^3 74 / 75, 64^3 133 / 130, 72^3 153 / 162, 80^3 194 / 242, 96^3 284 / 398, 160x20x20 57 / 60.
+// Near the crossing the estimate can take the slower form by a few percent (64^3: the single pass).
 inline bool march_pays(const DevParams &p, int cus) {
   const double tiles =
       (double)((p.nx + kMarchOutX - 1) / kMarchOutX) * ((p.ny + kMarchOutY - 1) / kMarchOutY);

@@ -13,10 +13,10 @@ namespace march2k {
 
 // One wave per strip (or pair of 32-column strips), four waves per block that do not interact.
 // Bound by instruction issue (about 1,460 FP64 and 400 other instructions per row and wave, 4
-// cycles each, reciprocals and square roots 16): two waves per SIMD at 256 registers (none
-// spilled) take 1.9 times the time of one.  Measured per launch: 2048^2 0.294 ms (14.3 G
-// cell-updates/s), where the three-kernel form's kernels took 0.890 ms, 1024^2 95 us, 256^2 23 us,
-// 64^2 15 us.  HBM traffic 168 bytes per cell (the state once each way is 128).
+// cycles each, reciprocals and square roots 16): two waves per SIMD at 256 registers (2
+// spilled) take 1.9 times the time of one.  Measured per launch: 2048^2 0.287 ms (14.6 G
+// cell-updates/s), where the three-kernel form's kernels take 0.875 ms, 1024^2 87 us, 256^2 23 us,
+// 64^2 16 us.  HBM traffic 168 bytes per cell (the state once each way is 128).
 // RS, ST, ISO: as k_march3d (Riemann solver; minmod factor fixed; isothermal branches).
 template <int RS, int ST, int ISO>
 __global__ void __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(2, 2)))

@@ -1,4 +1,4 @@
-// Single-pass 2D MHD step (k_march2d, and the 2D stage of the batch): the program of one wave.
+// Single-pass 2D MHD step (k_march2d): the program of one wave.
 //
 // A wave holds 64 / LW strips of LW columns (LW = 64: one strip, LW = 32: two strips side by
 // side in its lanes) and marches along y, one row per pass.  The middle LW - 4 columns of a
@@ -52,7 +52,8 @@ __device__ __forceinline__ double from_right(double x) { return __shfl_down(x, 1
 // Fix a value in its register, as a value read from memory is: the compiler neither contracts
 // its product into the sums of its users nor keeps its operands alive for that.  Applied to the
 // values that the three-kernel form passes through LDS and HBM, it rounds nearly as that form
-// does and took the spills of k_march2d from 17 to 6 registers (2048^2: 364 -> 337 us).
+// does and took the spills of k_march2d from 17 to 6 registers (2048^2: 364 -> 337 us; with the
+// leaner solvers 2 are spilled).
 __device__ __forceinline__ void settle(double &x) { asm volatile("" : "+v"(x)); }
 __device__ __forceinline__ void settle(St<double> &s) {
 #pragma unroll

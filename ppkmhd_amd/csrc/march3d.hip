@@ -30,7 +30,7 @@ struct DevExec {
 
 // One block per CU, marching its share of the grid's tile-planes (tiles of 18 x 14 record
 // columns); 4 waves, one block per CU (the LDS of one block is 152 KB), one wave per SIMD with
-// up to 512 registers.  Bound by instruction issue at that one wave: 256^3 in 4.55 ms (4.95
+// up to 512 registers.  Bound by instruction issue at that one wave: 256^3 in 4.58 ms (4.95
 // before the leaner solvers and the scalar load bases), 0.95 TB/s of HBM traffic.
 // RS: Riemann solver; ST: 1 for minmod slopes with the factor fixed, 0 to read slope_type;
 // ISO: 0 when the equation of state is not isothermal (cIso <= 0), so that the isothermal

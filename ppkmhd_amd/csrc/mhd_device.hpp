@@ -80,8 +80,9 @@ constexpr bool kSharedRecip = true;
 #endif
 // The default build's solvers (kLean) take forms that need fewer square roots and quotients
 // than the reference's expressions; each such place says which.  PPK_KEEP_ROUNDING (the batched
-// kernels) leaves them out: a long ensemble amplifies last-bit differences of a step until two
-// builds of the library disagree in 11 digits, and ensembles are kept to be compared.
+// kernels, in PPK_FP64 and PPK_FP32_BULK) leaves them out, so that a batch member and a single
+// grid of the same parameters differ by roundoff: a long ensemble amplifies the last bits of a step
+// (1e-11 after 400 steps), and its results stay those of the library's earlier builds.
 #ifdef PPK_KEEP_ROUNDING
 constexpr bool kLean = false;
 #else

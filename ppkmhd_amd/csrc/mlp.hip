@@ -24,7 +24,8 @@ using namespace mlpd;
 
 constexpr int kWaveSamples = 64;  // inference: samples per wavefront
 constexpr int kTrainWaves = 8, kGroup = 16 * kTrainWaves;  // k_train: samples per pass of a block
-constexpr int kMaxTrainBlocks = 256;  // one per CU; more groups are walked with this stride
+constexpr int kMaxTrainBlocks = 256;  // the CUs of an MI355X, on any device, so that the order of
+                                      // the sums is the same; more groups are walked with this stride
 constexpr int kAdamParts = 4;  // k_adam: most threads per parameter
 // row stride of the feature-major LDS arrays: 8 samples more than a group, so that the 16 rows
 // of an operand load start 4 banks apart
