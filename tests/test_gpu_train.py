@@ -53,3 +53,18 @@ def test_packed_copies_follow_training(gpu):
     fresh.set_params(net.get_params())
     assert np.array_equal(net.infer(X), fresh.infer(X))
     assert np.array_equal(net.gradient(X[:512], T[:512]), fresh.gradient(X[:512], T[:512]))
+
+
+@pytest.mark.parametrize("batch", [256, 4096, 33024])
+def test_training_repeats_itself(gpu, batch):
+    """The order of every sum is fixed: the same training gives the same bits."""
+    S, _, X, T = net_and_samples(40000)
+    fs = S.FaceSet(40000)
+    fs.append(X, T)
+    out = []
+    for _ in range(2):
+        net = S.MLP(5)
+        net.standardize(fs)
+        net.train(fs, 20, batch=batch, lr=1e-3, seed=3)
+        out.append(net.get_params())
+    assert np.array_equal(*out)
